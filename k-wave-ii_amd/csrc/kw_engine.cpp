@@ -331,8 +331,26 @@ struct Group {
       dirty = false;
       return;
     }
+    // a fixed-length variant serves the launch only if every member has
+    // that length on the pass's axis
+    auto common = [&](auto len, PassKind kind) -> int {
+      const int N = len(*sims[0]);
+      for (Sim* s : sims)
+        if (len(*s) != N) return 0;
+      return std::getenv("KW_NO_FIXED") ? 0 : fixed_variant(N, kind);
+    };
+    fixed[0] = common([](const Sim& s) { return s.G.Nx; }, PK_X_GRAD);
+    fixed[1] = dim == 3 ? common([](const Sim& s) { return s.G.Ny; }, PK_YFWD) : 0;
+    fixed[2] = common([&](const Sim& s) { return dim == 3 ? s.G.Nz : s.G.Ny; }, PK_SPEC);
     std::vector<ProbDev> hp(n);
-    for (int i = 0; i < n; ++i) hp[i] = sims[i]->P;
+    for (int i = 0; i < n; ++i) {
+      hp[i] = sims[i]->P;
+      // threads per pencil of the engine that serves the launch
+      const Geometry& g = sims[i]->G;
+      const int Nl = dim == 3 ? g.Nz : g.Ny;
+      hp[i].Gl = fixed[2] ? strided_threads(Nl) : rt_threads(Nl);
+      if (dim == 3) hp[i].Gy = fixed[1] ? strided_threads(g.Ny) : rt_threads(g.Ny);
+    }
     probs = (ProbDev*)dev_alloc(sizeof(ProbDev) * n);
     live.push_back(probs);
     dev_h2d(probs, hp.data(), sizeof(ProbDev) * n, stream);
@@ -349,7 +367,7 @@ struct Group {
         const LaunchGeom& g = geom_of(*sims[i], k);
         start[i] = (int32_t)nb;
         nb += g.nb;
-        T = std::max(T, g.T);
+        T = std::max(T, k == GL ? hp[i].Pl * hp[i].Gl : k == GY ? hp[i].Py * hp[i].Gy : g.T);
       }
       if (nb >= INT32_MAX) fail(KW_EUNSUP, "too many blocks in one group launch");
       // a block has T threads for every member: an x pass member gives each
@@ -371,17 +389,6 @@ struct Group {
       live.push_back(tiles[k]);
       dev_h2d(tiles[k], start.data(), sizeof(int32_t) * n, stream);
     }
-    // a fixed-length variant serves the launch only if every member has
-    // that length on the pass's axis
-    auto common = [&](auto len, PassKind kind) -> int {
-      const int N = len(*sims[0]);
-      for (Sim* s : sims)
-        if (len(*s) != N) return 0;
-      return std::getenv("KW_NO_FIXED") ? 0 : fixed_variant(N, kind);
-    };
-    fixed[0] = common([](const Sim& s) { return s.G.Nx; }, PK_X_GRAD);
-    fixed[1] = dim == 3 ? common([](const Sim& s) { return s.G.Ny; }, PK_YFWD) : 0;
-    fixed[2] = common([&](const Sim& s) { return dim == 3 ? s.G.Nz : s.G.Ny; }, PK_SPEC);
     any_points = any_grid = false;
     for (Sim* s : sims) {
       any_points = any_points || s->P.rec_points != 0;
@@ -397,9 +404,10 @@ struct Group {
     const int fx = fixed[k == GX ? 0 : (k == GY ? 1 : 2)];
     PassArgs a = a0;
     int nb = geo[k].nb;
-    if (k == GY && a.nbuf > 1 && ysplit_on()) {
+    const int split = split_buffers(kind, a, dim, (int64_t)nb * geo[k].T);
+    if (split > 1) {
       a.ysplit = nb;
-      nb *= a.nbuf;
+      nb *= split;
     }
     launch_pass(kind, fx, dim, nb, geo[k].T, launch_lds(kind, fx, a, geo[k].lds), batch(k), a,
                 stream);

@@ -32,6 +32,8 @@
 // once to float.  No normalisation is applied in either direction.
 #pragma once
 
+#include <type_traits>
+
 #include "kw_common.h"
 
 namespace kw {
@@ -53,30 +55,74 @@ struct FftPlan {
   const cf* bspec;  // Bluestein only: transform of the chirp filter, L entries
 };
 
-// factorisation rule shared by the host planner and the compile-time plans:
-// radix-8 stages first, then one radix-4 or radix-2 stage, then 3s and 5s
-constexpr int ct_nst(int N) {
-  int n = N, c = 0;
-  while (n % 8 == 0) { n /= 8; ++c; }
-  if (n % 4 == 0) { n /= 4; ++c; }
-  if (n % 2 == 0) { n /= 2; ++c; }
-  while (n % 3 == 0) { n /= 3; ++c; }
-  while (n % 5 == 0) { n /= 5; ++c; }
-  return n == 1 ? c : -1;
+// ---- compile-time plans -----------------------------------------------------
+// The stages of a fixed length.  A stage costs a thread its elements and, in
+// LDS round trip, barrier and index arithmetic, about kStageCost more; the plan
+// has the least of that over all radix sequences (486: 9 9 6 for six stages of
+// radix 2 and 3).
+struct CtPlan {
+  int nst = 0;
+  int r[KW_MAX_STAGES] = {};
+  int cost = 1 << 30;
+};
+constexpr int kStageCost = 3;
+
+// elements of one stage of radix R per thread
+constexpr int ct_stage_work(int N, int R, int G) { return (N / R + G - 1) / G * R; }
+
+constexpr void ct_search(int N, int rest, int G, int emax, CtPlan cur, int cost, int top,
+                         CtPlan& best) {
+  if (rest == 1) {
+    if (cur.nst > 0 && cost < best.cost) {
+      best = cur;
+      best.cost = cost;
+    }
+    return;
+  }
+  if (cost >= best.cost || cur.nst >= 8) return;
+  const int radices[9] = {12, 10, 9, 8, 6, 5, 4, 3, 2};
+  for (int i = 0; i < 9; ++i) {
+    const int R = radices[i];
+    if (R > top || rest % R != 0) continue;
+    const int w = ct_stage_work(N, R, G);
+    if (w > emax) continue;
+    CtPlan nx = cur;
+    nx.r[nx.nst++] = R;
+    ct_search(N, rest / R, G, emax, nx, cost + w + kStageCost, R, best);
+  }
 }
-constexpr int ct_radix(int N, int s) {
-  int n = N, c = 0;
-  while (n % 8 == 0) { n /= 8; if (c++ == s) return 8; }
-  if (n % 4 == 0) { n /= 4; if (c++ == s) return 4; }
-  if (n % 2 == 0) { n /= 2; if (c++ == s) return 2; }
-  while (n % 3 == 0) { n /= 3; if (c++ == s) return 3; }
-  while (n % 5 == 0) { n /= 5; if (c++ == s) return 5; }
-  return 0;
+
+// strided plan of length N with G threads, largest radix first (the first
+// stage has no twiddles)
+constexpr CtPlan ct_strided(int N, int G) {
+  CtPlan best;
+  ct_search(N, N, G, 12, CtPlan{}, 0, 12, best);
+  return best;
 }
-// product of the radices before stage s
-constexpr int ct_ns(int N, int s) {
-  int p = 1;
-  for (int i = 0; i < s; ++i) p *= ct_radix(N, i);
+// threads per pencil of the strided plan: the least work over all lanes,
+// then the most threads
+constexpr int strided_threads(int N) {
+  int g = 0, work = 1 << 30;
+  for (int G = (N + 11) / 12; G <= (N + 7) / 8; ++G) {
+    const CtPlan p = ct_strided(N, G);
+    if (p.nst > 0 && p.cost * G <= work) {
+      g = G;
+      work = p.cost * G;
+    }
+  }
+  return g;
+}
+// x plan: the stage that leaves a thread the fewest elements last, the
+// largest of the others first
+constexpr CtPlan ct_xplan(int N, int G) {
+  CtPlan p;
+  ct_search(N, N, G, 12, CtPlan{}, 0, 10, p);
+  int last = 0;
+  for (int s = 1; s < p.nst; ++s)
+    if (ct_stage_work(N, p.r[s], G) <= ct_stage_work(N, p.r[last], G)) last = s;
+  const int R = p.r[last];
+  for (int s = last; s + 1 < p.nst; ++s) p.r[s] = p.r[s + 1];
+  if (p.nst > 0) p.r[p.nst - 1] = R;
   return p;
 }
 
@@ -100,7 +146,7 @@ static_assert(MaxB<2>::v * 2 <= kMaxSlots && MaxB<3>::v * 3 <= kMaxSlots &&
 
 // Twiddle table of a plan as the stages read it: in HBM (each read a vector
 // memory load through the same address path as the data streams), or
-// copied once per block into LDS (stage_twiddles).
+// copied once per block into LDS (put_twiddles).
 struct TwG {
   const cf* p;
 };
@@ -122,12 +168,34 @@ KW_BODY cf twiddle(const TwL& tw, int idx) {
 }
 
 // the L twiddles of a plan copied into the block's LDS at `dst` by all
-// threads of the block, followed by a block barrier
+// threads of the block (the caller synchronises), four loads in flight per
+// thread: a small tile has fewer threads than twiddles, and one load at a
+// time would cost it a memory latency per round
 template <class Ctx>
-KW_BODY TwL stage_twiddles(Ctx& c, const FftPlan& pl, cf* dst) {
-  for (int i = c.tid(); i < pl.L; i += c.nthreads()) lds_st(dst + i, KW_LD32(pl.tw, (uint32_t)i));
-  c.sync();
+KW_BODY TwL put_twiddles(Ctx& c, const FftPlan& pl, cf* dst) {
+  const int L = pl.L, nt = c.nthreads();
+  for (int i = c.tid(); i < L; i += 4 * nt) {
+    cf w[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int n = i + k * nt;
+      w[k] = KW_LD32(pl.tw, (uint32_t)(n < L ? n : i));
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (i + k * nt < L) lds_st(dst + i + k * nt, w[k]);
+  }
   return TwL{dst};
+}
+
+// value of input n (slot: its place among the calling thread's inputs of
+// the first stage), from a source that takes the slot or one that does not
+template <class Src>
+KW_BODY cf fetch(Src& src, int j, int n, int slot) {
+  if constexpr (std::is_invocable_v<Src&, int, int, int>)
+    return src(j, n, slot);
+  else
+    return src(j, n);
 }
 
 // radix-R DFT in place; forward uses exp(-2 pi i rs/R), inverse exp(+...)
@@ -269,6 +337,73 @@ KW_BODY void dft<8, false>(cf* v) { dft8<false>(v); }
 template <>
 KW_BODY void dft<8, true>(cf* v) { dft8<true>(v); }
 
+// radix A B with A and B coprime by the prime-factor map (no twiddles):
+// input (B i + A j) mod AB, output k with k = i' mod A and k = j' mod B
+template <int A, int B, bool INV>
+KW_BODY void dft_pfa(cf* v) {
+  constexpr int R = A * B;
+  cf t[B][A];
+#pragma unroll
+  for (int j = 0; j < B; ++j) {
+#pragma unroll
+    for (int i = 0; i < A; ++i) t[j][i] = v[(B * i + A * j) % R];
+    dft<A, INV>(t[j]);
+  }
+  // after the A transforms column i holds B values per output i
+#pragma unroll
+  for (int i = 0; i < A; ++i) {
+    cf w[B];
+#pragma unroll
+    for (int j = 0; j < B; ++j) w[j] = t[j][i];
+    dft<B, INV>(w);
+#pragma unroll
+    for (int k = 0; k < R; ++k)
+      if (k % A == i) v[k] = w[k % B];
+  }
+}
+template <> KW_BODY void dft<6, false>(cf* v) { dft_pfa<3, 2, false>(v); }
+template <> KW_BODY void dft<6, true>(cf* v) { dft_pfa<3, 2, true>(v); }
+template <> KW_BODY void dft<10, false>(cf* v) { dft_pfa<5, 2, false>(v); }
+template <> KW_BODY void dft<10, true>(cf* v) { dft_pfa<5, 2, true>(v); }
+template <> KW_BODY void dft<12, false>(cf* v) { dft_pfa<3, 4, false>(v); }
+template <> KW_BODY void dft<12, true>(cf* v) { dft_pfa<3, 4, true>(v); }
+
+// multiply by exp(-+ i angle) given its cosine and sine
+template <bool INV>
+KW_BODY cf cturn(cf a, float co, float si) {
+  return INV ? cmul(a, cf{co, si}) : cmul(a, cf{co, -si});
+}
+
+// radix 9 as 3 x 3: input 3 n1 + n2, output k1 + 3 k2, constant twiddles
+// between
+template <bool INV>
+KW_BODY void dft9(cf* v) {
+  // cos and sin of 2 pi j / 9, j = 1, 2, 4
+  const float c1 = 0.766044443118978f, s1 = 0.6427876096865393f;
+  const float c2 = 0.17364817766693036f, s2 = 0.984807753012208f;
+  const float c4 = -0.9396926207859084f, s4 = 0.3420201433256687f;
+  cf t[3][3];
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+#pragma unroll
+    for (int j = 0; j < 3; ++j) t[i][j] = v[3 * j + i];
+    dft<3, INV>(t[i]);
+  }
+  t[1][1] = cturn<INV>(t[1][1], c1, s1);
+  t[1][2] = cturn<INV>(t[1][2], c2, s2);
+  t[2][1] = cturn<INV>(t[2][1], c2, s2);
+  t[2][2] = cturn<INV>(t[2][2], c4, s4);
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    cf w[3] = {t[0][k], t[1][k], t[2][k]};
+    dft<3, INV>(w);
+#pragma unroll
+    for (int m = 0; m < 3; ++m) v[k + 3 * m] = w[m];
+  }
+}
+template <> KW_BODY void dft<9, false>(cf* v) { dft9<false>(v); }
+template <> KW_BODY void dft<9, true>(cf* v) { dft9<true>(v); }
+
 KW_BODY int mod_ns(int b, int Ns) {
   // b mod Ns; Ns is a compile-time constant in the fixed-length engine and
   // a power of two for every stage before the first radix-3/5 stage
@@ -301,7 +436,7 @@ KW_BODY void stage(Ctx& c, int N, int Ns, int G, int g, bool active, const TW& t
 #pragma unroll
       for (int j = 0; j < NP; ++j) {
 #pragma unroll
-        for (int r = 0; r < R; ++r) v[j][m][r] = src(j, b + r * nb);
+        for (int r = 0; r < R; ++r) v[j][m][r] = fetch(src, j, b + r * nb, m * R + r);
       }
 #pragma unroll
       for (int j = 0; j < NP; ++j) {
@@ -477,50 +612,82 @@ KW_BODY void last_slots_rt(const FftPlan& pl, int g, int G, bool, F& f) {
 
 // ---- fixed-length engine ------------------------------------------------------
 
-template <int N, int G, int S, int NST, int NP, bool INV>
+// N, threads per pencil G and the plan family (X: x passes) as constants
+template <int N_, int G_, bool X>
+struct CtShape {
+  static constexpr int N = N_;
+  static constexpr int G = G_;
+  static constexpr CtPlan plan = X ? ct_xplan(N, G) : ct_strided(N, G);
+  static constexpr int nst = plan.nst;
+  static_assert(nst > 0, "length must factor into 2, 3 and 5");
+  static constexpr int radix(int s) { return plan.r[s]; }
+  static constexpr int ns(int s) {
+    int p = 1;
+    for (int i = 0; i < s; ++i) p *= plan.r[i];
+    return p;
+  }
+  static constexpr int mb(int s) { return (N / plan.r[s] + G - 1) / G; }
+  // inputs of the first and outputs of the last stage per thread
+  static constexpr int first_slots = mb(0) * plan.r[0];
+  static constexpr int last_slots = mb(nst - 1) * plan.r[nst - 1];
+};
+
+template <class Sh, int S, int NP, bool INV>
 struct CtStages {
-  static constexpr int R = ct_radix(N, S);
-  static constexpr int Ns = ct_ns(N, S);
-  static constexpr int MB = (N / R + G - 1) / G;
+  static constexpr int R = Sh::radix(S);
+  static constexpr int Ns = Sh::ns(S);
+  static constexpr int MB = Sh::mb(S);
   template <class Ctx, class TW, class Src, class Dst, class LSrc, class LDst>
   KW_BODY static void run(Ctx& c, int g, bool active, const TW& tw, Src& src0, Dst& dstN,
                           LSrc& lsrc, LDst& ldst) {
-    if constexpr (S == 0 && NST == 1) {
-      stage<R, NP, INV, MB>(c, N, Ns, G, g, active, tw, src0, dstN);
+    if constexpr (S == 0 && Sh::nst == 1) {
+      stage<R, NP, INV, MB>(c, Sh::N, Ns, Sh::G, g, active, tw, src0, dstN);
     } else if constexpr (S == 0) {
-      stage<R, NP, INV, MB>(c, N, Ns, G, g, active, tw, src0, ldst);
-    } else if constexpr (S == NST - 1) {
-      stage<R, NP, INV, MB>(c, N, Ns, G, g, active, tw, lsrc, dstN);
+      stage<R, NP, INV, MB>(c, Sh::N, Ns, Sh::G, g, active, tw, src0, ldst);
+    } else if constexpr (S == Sh::nst - 1) {
+      stage<R, NP, INV, MB>(c, Sh::N, Ns, Sh::G, g, active, tw, lsrc, dstN);
     } else {
-      stage<R, NP, INV, MB>(c, N, Ns, G, g, active, tw, lsrc, ldst);
+      stage<R, NP, INV, MB>(c, Sh::N, Ns, Sh::G, g, active, tw, lsrc, ldst);
     }
-    if constexpr (S + 1 < NST)
-      CtStages<N, G, S + 1, NST, NP, INV>::run(c, g, active, tw, src0, dstN, lsrc, ldst);
+    if constexpr (S + 1 < Sh::nst)
+      CtStages<Sh, S + 1, NP, INV>::run(c, g, active, tw, src0, dstN, lsrc, ldst);
   }
 };
 
-template <int N, int G, int NP, bool INV, class Ctx, class TW, class Src, class Dst>
+template <class Sh, int NP, bool INV, class Ctx, class TW, class Src, class Dst>
 KW_BODY void fft_ct(Ctx& c, const TW& tw, int g, bool active, Src& src0, Dst& dstN,
                     const LdsPencils& lds) {
-  static_assert(ct_nst(N) > 0, "length must factor into 2, 3 and 5");
   g = kw_fresh(g);
   auto lsrc = [&](int j, int n) -> cf { return lds.get(j, n); };
   auto ldst = [&](int j, int n, cf v, int) { lds.set(j, n, v); };
-  CtStages<N, G, 0, ct_nst(N), NP, INV>::run(c, g, active, tw, src0, dstN, lsrc, ldst);
+  CtStages<Sh, 0, NP, INV>::run(c, g, active, tw, src0, dstN, lsrc, ldst);
 }
 
-template <int N, int G, class F>
-KW_BODY void last_slots_ct(int g, bool, F& f) {
-  constexpr int S = ct_nst(N) - 1;
-  constexpr int R = ct_radix(N, S);
-  constexpr int Ns = N / R;
-  constexpr int nb = N / R;
-  constexpr int MB = (nb + G - 1) / G;
+// f(slot, n) for this thread's inputs of the first stage, in the order the
+// stage reads them
+template <class Sh, class F>
+KW_BODY void first_slots_ct(int g, F& f) {
+  constexpr int R = Sh::radix(0), nb = Sh::N / R, MB = Sh::mb(0);
   g = kw_fresh(g);
 #pragma unroll
   for (int m = 0; m < MB; ++m) {
-    const int b = g + m * G;
-    if (MB * G == nb || b < nb) {
+    const int b = g + m * Sh::G;
+    if (MB * Sh::G == nb || b < nb) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) f(m * R + r, b + r * nb);
+    }
+  }
+}
+
+template <class Sh, class F>
+KW_BODY void last_slots_ct(int g, bool, F& f) {
+  constexpr int S = Sh::nst - 1;
+  constexpr int R = Sh::radix(S), Ns = Sh::ns(S), nb = Sh::N / R, MB = Sh::mb(S);
+  g = kw_fresh(g);
+#pragma unroll
+  for (int m = 0; m < MB; ++m) {
+    const int b = g + m * Sh::G;
+    if (MB * Sh::G == nb || b < nb) {
       const int k = mod_ns(b, Ns);
       const int j0 = (b - k) * R + k;
 #pragma unroll
@@ -533,15 +700,42 @@ KW_BODY void last_slots_ct(int g, bool, F& f) {
 // A kernel body templated on a selector runs the runtime engine (PlanRt) or
 // the fixed-length engine (PlanCt<N>) for one axis.
 
+// What a source's first loads bring into registers and how an input is made
+// of it: sources that combine several loads name a Raw type and give raw(n)
+// and join(raw, n), so that the loads can be in flight before the combination
+// waits for them; any other source is called.
+template <class Src, class = void>
+struct SrcRaw {
+  using type = cf;
+  KW_BODY static cf raw(Src& s, int n) { return s(0, n); }
+  KW_BODY static cf join(Src&, const cf& r, int) { return r; }
+};
+template <class Src>
+struct SrcRaw<Src, std::void_t<typename Src::Raw>> {
+  using type = typename Src::Raw;
+  KW_BODY static type raw(Src& s, int n) { return s.raw(n); }
+  KW_BODY static cf join(Src& s, const type& r, int n) { return s.join(r, n); }
+};
+
+// Start of a block: `load_first` issues the loads of a transform's first
+// stage before the block has its twiddles, which that stage does not use, so
+// the two memory latencies overlap; `fft_pre` runs the transform from them.
+
 struct PlanRt {
   static constexpr int fixed = 0;
   static constexpr int G = 0;  // threads per pencil: chosen at run time
-  template <int NP, bool INV, class Ctx, class Src, class Dst>
-  KW_BODY static void fft(Ctx& c, const FftPlan& pl, int g, int G, bool active, Src& src,
-                          Dst& dst, const LdsPencils& lds) {
-    fft_rt<NP, INV>(c, pl, TwG{pl.tw}, g, G, active, src, dst, lds);
+  template <class Src>
+  struct Pre {};
+  template <class Src>
+  KW_BODY static void load_first(int, Src&, Pre<Src>&) {}
+  // the runtime stages start from LDS, so the block's twiddles are waited
+  // for before anything else
+  static constexpr bool twiddles_first = true;
+  template <int NP, bool INV, class Ctx, class TW, class Src, class Dst>
+  KW_BODY static void fft_pre(Ctx& c, const FftPlan& pl, const TW& tw, int g, int G, bool active,
+                              Src& src, Pre<Src>&, Dst& dst, const LdsPencils& lds) {
+    fft_rt<NP, INV>(c, pl, tw, g, G, active, src, dst, lds);
   }
-  // the same with the twiddles read from `tw` (for example staged in LDS)
   template <int NP, bool INV, class Ctx, class TW, class Src, class Dst>
   KW_BODY static void fft_tw(Ctx& c, const FftPlan& pl, const TW& tw, int g, int G, bool active,
                              Src& src, Dst& dst, const LdsPencils& lds) {
@@ -553,47 +747,66 @@ struct PlanRt {
   }
 };
 
-// threads per pencil of a fixed-length plan: ceil(N / KW_E)
+// threads per pencil of the runtime engine: ceil(N / KW_E)
 KW_HOSTDEV constexpr int ct_threads(int N) { return (N + KW_E - 1) / KW_E; }
 
-// threads per pencil of the fixed-length x passes: ceil(N / KW_E) rounded up
-// to a power of two when that is at most 64, so that every pencil lies in
-// one wavefront and the stages synchronise with wavefront barriers instead
-// of block barriers (the extra lanes idle in stages with fewer butterflies
-// than lanes)
+// threads per pencil of the fixed-length x passes: the smallest power of two
+// that leaves a thread at most six elements, so that every pencil lies in one
+// wavefront and the stages synchronise with wavefront barriers instead of
+// block barriers (the extra lanes idle in stages with fewer butterflies than
+// lanes); lengths above 384 take ceil(N / KW_E)
 KW_HOSTDEV constexpr int x_threads(int N) {
-  int g = ct_threads(N), p = 1;
-  if (g > 64) return g;
-  while (p < g) p <<= 1;
-  return p;
+  for (int p = 1; p <= 64; p <<= 1)
+    if (6 * p >= N) return p;
+  return ct_threads(N) <= 64 ? 64 : ct_threads(N);
 }
 
-template <int N_, int G_ = ct_threads(N_)>
-struct PlanCt {
-  static constexpr int fixed = N_;
+template <class Sh>
+struct PlanFixed {
+  static constexpr int fixed = Sh::N;
   // threads per pencil; when N is not a multiple of G some threads get
   // fewer butterflies (the stages guard them)
-  static constexpr int G = G_;
-  static constexpr int last_R = ct_radix(N_, ct_nst(N_) - 1);
-  static_assert(((N_ / last_R + G - 1) / G) * last_R <= kMaxSlots, "slot bound");
-  template <int NP, bool INV, class Ctx, class Src, class Dst>
-  KW_BODY static void fft(Ctx& c, const FftPlan& pl, int g, int, bool active, Src& src, Dst& dst,
-                          const LdsPencils& lds) {
-    fft_ct<N_, G, NP, INV>(c, TwG{pl.tw}, g, active, src, dst, lds);
+  static constexpr int G = Sh::G;
+  // with one stage there is no block barrier between the twiddles and their
+  // first use (and no twiddle is used)
+  static constexpr bool twiddles_first = false;
+  template <class Src>
+  struct Pre {
+    typename SrcRaw<Src>::type v[Sh::first_slots];
+  };
+  template <class Src>
+  KW_BODY static void load_first(int g, Src& src, Pre<Src>& pre) {
+    auto f = [&](int slot, int n) { pre.v[slot] = SrcRaw<Src>::raw(src, n); };
+    first_slots_ct<Sh>(g, f);
+  }
+  template <int NP, bool INV, class Ctx, class TW, class Src, class Dst>
+  KW_BODY static void fft_pre(Ctx& c, const FftPlan&, const TW& tw, int g, int, bool active,
+                              Src& src, Pre<Src>& pre, Dst& dst, const LdsPencils& lds) {
+    static_assert(NP == 1, "one pencil");
+    auto held = [&](int, int n, int slot) -> cf {
+      return SrcRaw<Src>::join(src, pre.v[slot], n);
+    };
+    fft_ct<Sh, 1, INV>(c, tw, g, active, held, dst, lds);
   }
   template <int NP, bool INV, class Ctx, class TW, class Src, class Dst>
   KW_BODY static void fft_tw(Ctx& c, const FftPlan&, const TW& tw, int g, int, bool active,
                              Src& src, Dst& dst, const LdsPencils& lds) {
-    fft_ct<N_, G, NP, INV>(c, tw, g, active, src, dst, lds);
+    fft_ct<Sh, NP, INV>(c, tw, g, active, src, dst, lds);
   }
   template <class F>
   KW_BODY static void last_slots(const FftPlan&, int g, int, bool active, F& f) {
-    last_slots_ct<N_, G>(g, active, f);
+    last_slots_ct<Sh>(g, active, f);
   }
 };
 
+// the plan of the strided and last-axis passes for a fixed length
+template <int N>
+using PlanCt = PlanFixed<CtShape<N, strided_threads(N), false>>;
+
 // the plan of the x passes for a fixed length
 template <int N>
-using PlanCtX = PlanCt<N, x_threads(N)>;
+struct PlanCtX : PlanFixed<CtShape<N, x_threads(N), true>> {
+  static_assert(CtShape<N, x_threads(N), true>::last_slots <= kMaxSlots, "slot bound");
+};
 
 }  // namespace kw

@@ -96,12 +96,20 @@ KW_BODY XTile x_tile(Ctx& c, const ProbDev& P, int tile) {
   T.z0 = r0 / (uint32_t)P.Ny;
   T.y1 = r1 % (uint32_t)P.Ny;
   T.z1 = r1 / (uint32_t)P.Ny;
-  // LDS: the L twiddles of the x transform (staged by the whole block), then
-  // the pencils (L elements each, padded)
-  T.tw = stage_twiddles(c, P.fx, c.lds());
+  // LDS: the L twiddles of the x transform (put there by x_start), then the
+  // pencils (L elements each, padded)
+  T.tw = TwL{c.lds()};
   const int stride = x_lds_stride(P.fx.L);
   T.lds = LdsPencils{c.lds() + P.fx.L + (int64_t)p * kNPX * stride, stride, 1, true};
   return T;
+}
+
+// the twiddles into LDS and the block barrier that makes them visible to
+// every wavefront; the caller has issued its first loads before
+template <class Ctx>
+KW_BODY void x_start(Ctx& c, const ProbDev& P) {
+  put_twiddles(c, P.fx, c.lds());
+  c.sync();
 }
 
 // LDS pencil j holds Z = fft(a + i b) in natural order; split into the half
@@ -138,20 +146,22 @@ KW_BODY void x_fwd_from_lds(Ctx& c, const ProbDev& P, const XTile& T, cf* const*
 
 // inverse two-for-one load functor: Z_j[n] = A_j[n] + i B_j[n]; row r1 is
 // r0 when the pair has a single row (the B part is then zeroed by select)
-template <int NP>
 struct HalfPairLoad {
   const ProbDev* P;
-  const cf* S[NP];
+  const cf* S;
   uint32_t h0, h1, q0, q1;
   bool has1;
-  KW_BODY cf operator()(int j, int n) const {
-    const cf a = half_get(*P, S[j], h0, q0, n);
-    cf b = half_get(*P, S[j], h1, q1, n);
+  KW_BODY cf operator()(int, int n) const {
+    const cf a = half_get(*P, S, h0, q0, n);
+    cf b = half_get(*P, S, h1, q1, n);
     b.x = has1 ? b.x : 0.f;
     b.y = has1 ? b.y : 0.f;
     return cf{a.x - b.y, a.y + b.x};
   }
 };
+KW_BODY HalfPairLoad half_pair(const ProbDev& P, const XTile& T, const cf* S) {
+  return HalfPairLoad{&P, S, T.h0, T.h1, T.q0, T.q1, T.has1};
+}
 
 // 1-D PML factors of axis d for the two rows at x = n: x varies along the
 // row, y and z are constant along it
@@ -231,6 +241,21 @@ KW_BODY void x_source(const ProbDev& P, const XTile& T, const TimeSource& src, i
   });
 }
 
+// problem, tile and first buffer of a block whose launch has the tiles once
+// per buffer (A.ysplit tiles each; 0: every block does all buffers)
+template <class Ctx>
+KW_BODY const ProbDev& split_prob(Ctx& c, const Batch& B, const PassArgs& A, int& tile, int& b0) {
+  int vb = c.bid();
+  b0 = 0;
+  if (A.ysplit > 0) {
+    b0 = vb / A.ysplit;
+    vb -= b0 * A.ysplit;
+  }
+  const int pi = find_prob<Ctx>(B, vb);
+  tile = vb - KW_LD(B.tile_start + pi);
+  return B.probs[pi];
+}
+
 template <class Ctx>
 KW_BODY const ProbDev& batch_prob(Ctx& c, const Batch& B, int& tile) {
   const int pi = find_prob<Ctx>(B, c.bid());
@@ -249,22 +274,14 @@ KW_BODY void advance_step(const ProbDev& P, const PassArgs& A, int tile, int tid
 
 template <bool INV, class YS, class Ctx>
 KW_BODY void body_ypass(Ctx& c, const Batch& B, const PassArgs& A) {
-  // the launch's tiles, once per buffer when the buffers are split over
-  // blocks (ysplit), else every block loops over the buffers
-  int vb = c.bid(), b0 = 0, b1 = A.nbuf;
-  if (A.ysplit > 0) {
-    b0 = vb / A.ysplit;
-    b1 = b0 + 1;
-    vb -= b0 * A.ysplit;
-  }
-  const int pi = find_prob<Ctx>(B, vb);
-  const int tile = vb - KW_LD(B.tile_start + pi);
-  const ProbDev& P = B.probs[pi];
+  int tile, b0;
+  const ProbDev& P = split_prob(c, B, A, tile, b0);
+  const int b1 = A.ysplit > 0 ? b0 + 1 : A.nbuf;
   if (b0 == 0) advance_step(P, A, tile, c.tid());
   const int N = P.Ny, G = P.Gy, Pn = P.Py;
   // LDS: the L twiddles, then the pencils (L elements each: the length the
   // stages run at)
-  const TwL tw = stage_twiddles(c, P.fy, c.lds());
+  const TwL tw{c.lds()};
   const int L = P.fy.L;
   cf* const lp = c.lds() + L;
   const int64_t nH = (int64_t)P.Wm * P.Nz;
@@ -301,7 +318,16 @@ KW_BODY void body_ypass(Ctx& c, const Batch& B, const PassArgs& A) {
     cf* S = P.S[A.buf[b]];
     auto ld = [&](int, int n) -> cf { return KW_LD32(S, base + (uint32_t)n * stride); };
     auto st = [&](int, int n, cf v, int) { KW_ST32(S, base + (uint32_t)n * stride, v); };
-    YS::template fft_tw<1, INV>(c, P.fy, tw, g, G, active, ld, st, lds);
+    if (b == b0) {
+      // the first transform's loads are in flight while the twiddles come
+      typename YS::template Pre<decltype(ld)> pre;
+      YS::load_first(g, ld, pre);
+      put_twiddles(c, P.fy, c.lds());
+      if (YS::twiddles_first) c.sync();
+      YS::template fft_pre<1, INV>(c, P.fy, tw, g, G, active, ld, pre, st, lds);
+    } else {
+      YS::template fft_tw<1, INV>(c, P.fy, tw, g, G, active, ld, st, lds);
+    }
   }
 }
 
@@ -390,9 +416,10 @@ KW_HOSTDEV bool spec_is_aux(const PassArgs& A) { return A.mode == SM_SHIFT || A.
 // code.
 template <class LS, bool AUX, class Ctx>
 KW_BODY void body_spec(Ctx& c, const Batch& B, const PassArgs& A) {
-  int tile;
-  const ProbDev& P = batch_prob(c, B, tile);
-  advance_step(P, A, tile, c.tid());
+  // SM_DIV and SM_ABS with ysplit: one buffer per block
+  int tile, b0;
+  const ProbDev& P = split_prob(c, B, A, tile, b0);
+  if (b0 == 0) advance_step(P, A, tile, c.tid());
   const bool d3 = P.dim == 3;
   const FftPlan& pl = d3 ? P.fz : P.fy;
   const int N = pl.N, G = P.Gl, Pn = P.Pl;
@@ -431,7 +458,7 @@ KW_BODY void body_spec(Ctx& c, const Batch& B, const PassArgs& A) {
     ky = d3 ? 0 : -1;
   }
   // LDS: the L twiddles, then pencil buffers la and lb (L elements each)
-  const TwL tw = stage_twiddles(c, pl, c.lds());
+  const TwL tw{c.lds()};
   cf* const lp = c.lds() + pl.L;
   LdsPencils la{lp + p, 0, Pn, false};
   LdsPencils lb{lp + (int64_t)Pn * pl.L + p, 0, Pn, false};
@@ -457,13 +484,25 @@ KW_BODY void body_spec(Ctx& c, const Batch& B, const PassArgs& A) {
     la.set(0, n, cscale(v, KW_LD32(P.kappa, taddr(n))));
   };
 
+  // the block's first forward transform: its loads are in flight while the
+  // twiddles come
+  auto first = [&](auto& ld, auto& dst) {
+    typename LS::template Pre<std::remove_reference_t<decltype(ld)>> pre;
+    LS::load_first(g, ld, pre);
+    put_twiddles(c, pl, c.lds());
+    if (LS::twiddles_first) c.sync();
+    LS::template fft_pre<1, false>(c, pl, tw, g, G, active, ld, pre, dst, la);
+  };
+
   if constexpr (AUX) {
+    put_twiddles(c, pl, c.lds());
+    c.sync();
     spec_aux<LS>(c, P, A, pl, tw, N, G, last, g, active, tile, tH, kx, ky, la, lb, lw, addr, taddr,
                  to_a);
   } else if (A.mode == SM_GRAD) {
     cf* S0 = P.S[0];
     auto ld = [&](int, int n) -> cf { return KW_LD32(S0, addr(n)); };
-    LS::template fft_tw<1, false>(c, pl, tw, g, G, active, ld, to_ak, la);
+    first(ld, to_ak);
     // C = ifft(kappa .* S); x (and in 3D y) derivatives are per-pencil
     // constants times C
     const cf dx = active ? KW_LD(P.dpos[0] + kx) : cf{0.f, 0.f};
@@ -481,10 +520,13 @@ KW_BODY void body_spec(Ctx& c, const Batch& B, const PassArgs& A) {
     auto st2 = [&](int, int n, cf v, int) { KW_ST32(So, addr(n), v); };
     LS::template fft_tw<1, true>(c, pl, tw, g, G, active, src2, st2, lb);
   } else if (A.mode == SM_DIV) {
-    for (int d = 0; d < P.dim; ++d) {
+    for (int d = b0; d < (A.ysplit > 0 ? b0 + 1 : P.dim); ++d) {
       cf* S = P.S[d];
       auto ld = [&](int, int n) -> cf { return KW_LD32(S, addr(n)); };
-      LS::template fft_tw<1, false>(c, pl, tw, g, G, active, ld, to_ak, la);
+      if (d == b0)
+        first(ld, to_ak);
+      else
+        LS::template fft_tw<1, false>(c, pl, tw, g, G, active, ld, to_ak, la);
       const cf dc = (d == last || !active) ? cf{0.f, 0.f}
                                            : KW_LD(P.dneg[d] + (d == 0 ? kx : ky));
       const cf* dl = P.dneg[d];
@@ -497,12 +539,15 @@ KW_BODY void body_spec(Ctx& c, const Batch& B, const PassArgs& A) {
     }
   } else {
     // SM_ABS: S0 <- nabla1 .* S0, S1 <- nabla2 .* S1;  SM_FILTER: one table
-    const int nb = A.mode == SM_ABS ? 2 : 1;
-    for (int j = 0; j < nb; ++j) {
+    const int nb = A.ysplit > 0 ? b0 + 1 : A.mode == SM_ABS ? 2 : 1;
+    for (int j = b0; j < nb; ++j) {
       cf* S = P.S[A.mode == SM_ABS ? j : A.buf[0]];
       const float* tab = A.mode == SM_ABS ? (j == 0 ? P.nabla1 : P.nabla2) : A.table;
       auto ld = [&](int, int n) -> cf { return KW_LD32(S, addr(n)); };
-      LS::template fft_tw<1, false>(c, pl, tw, g, G, active, ld, to_a, la);
+      if (j == b0)
+        first(ld, to_a);
+      else
+        LS::template fft_tw<1, false>(c, pl, tw, g, G, active, ld, to_a, la);
       auto src = [&](int, int n) -> cf { return cscale(la.get(0, n), KW_LD32(tab, taddr(n))); };
       auto st = [&](int, int n, cf v, int) { KW_ST32(S, addr(n), v); };
       LS::template fft_tw<1, true>(c, pl, tw, g, G, active, src, st, lw);
@@ -520,6 +565,7 @@ KW_BODY void body_x_r2c(Ctx& cb, const Batch& B, const PassArgs& A) {
   int tile;
   const ProbDev& P = batch_prob(cb, B, tile);
   const XTile T = x_tile<XS>(cb, P, tile);
+  x_start(cb, P);
   PencilCtx<Ctx> c{cb, T.wave};
   // A.table: a factor per y row (the axisymmetric inverse radius), applied
   // as the rows are read
@@ -546,11 +592,12 @@ KW_BODY void body_x_c2r(Ctx& cb, const Batch& B, const PassArgs& A) {
   int tile;
   const ProbDev& P = batch_prob(cb, B, tile);
   const XTile T = x_tile<XS>(cb, P, tile);
+  x_start(cb, P);
   PencilCtx<Ctx> c{cb, T.wave};
   const bool acc = A.flags & XC_ACCUM;
   for (int b = 0; b < A.nbuf; ++b) {
     float* f = A.real[b];
-    HalfPairLoad<1> src{&P, {P.S[A.buf[b]]}, T.h0, T.h1, T.q0, T.q1, T.has1};
+    HalfPairLoad src = half_pair(P, T, P.S[A.buf[b]]);
     auto dst = [&](int, int n, cf v, int) {
       const uint32_t i0 = T.c0 + n, i1 = T.c1 + n;
       const float o0 = acc ? KW_LD32(f, i0) : 0.f;
@@ -566,7 +613,7 @@ KW_BODY void body_x_c2r(Ctx& cb, const Batch& B, const PassArgs& A) {
 // outputs gv[slot] (real parts: row r0, imaginary parts: row r1)
 template <class XS, class PC>
 KW_BODY void x_inverse(PC& c, const ProbDev& P, const XTile& T, const cf* S, cf* gv) {
-  HalfPairLoad<1> src{&P, {S}, T.h0, T.h1, T.q0, T.q1, T.has1};
+  HalfPairLoad src = half_pair(P, T, S);
   auto dst = [&](int, int, cf v, int slot) { gv[slot] = v; };
   KW_PHASE_FENCE();
   XS::template fft_tw<1, true>(c, P.fx, T.tw, T.g, T.G, T.active, src, dst, T.lds);
@@ -595,16 +642,19 @@ KW_BODY void x_forward(PC& c, const ProbDev& P, const XTile& T, const float* av,
 // u_d = dt rho0_sg_d^-1 g_d / 2 (:1023-1037), no fft.
 template <class XS, int DIM, class Ctx>
 KW_BODY void body_x_grad(Ctx& cb, const Batch& B, const PassArgs& A) {
-  int tile;
-  const ProbDev& P = batch_prob(cb, B, tile);
+  int tile, b0;
+  const ProbDev& P = split_prob(cb, B, A, tile, b0);
   const XTile T = x_tile<XS>(cb, P, tile);
   PencilCtx<Ctx> c{cb, T.wave};
   const int t = KW_LD(P.t_index);
   const bool init = A.flags & XG_INIT;
   const float dt = P.dt;
-  // one component at a time: inverse transform, update, forward transform
+  // one component at a time (one per block with ysplit): inverse transform,
+  // update, forward transform
+  const int b1 = A.ysplit > 0 ? b0 + 1 : DIM;
+  x_start(cb, P);
 #pragma unroll 1
-  for (int d = 0; d < DIM; ++d) {
+  for (int d = b0; d < b1; ++d) {
     cf gv[kMaxSlots];
     x_inverse<XS>(c, P, T, P.S[d], gv);
     float* u = P.u[d];
@@ -817,6 +867,7 @@ KW_BODY void body_x_div(Ctx& cb, const Batch& B, const PassArgs& A) {
   // and density; mass conservation coefficient k = rho0 (linear) or
   // 2 sum(rho) + rho0 (nonlinear, from the densities before this update),
   // kept in registers across the components
+  x_start(cb, P);
   float du0[kMaxSlots], du1[kMaxSlots], rs0[kMaxSlots], rs1[kMaxSlots];
   float k0[kMaxSlots], k1[kMaxSlots];
   // a single-series additive pressure source adds s(t) K_M to every density
@@ -945,6 +996,7 @@ KW_BODY void body_x_eos(Ctx& cb, const Batch& B, const PassArgs& A) {
   // rsum + tau A first, then - eta B and the nonlinear term; rsum is kept
   // across the second inverse only for the nonlinear term
   cf pv[kMaxSlots];
+  x_start(cb, P);
   with_flag(P.nonlinear != 0, [&](auto NL) {
     constexpr bool nl = decltype(NL)::value;
     cf part[kMaxSlots], rs[nl ? kMaxSlots : 1];

@@ -80,6 +80,14 @@ inline int stage_length(int N) {
   return factorise(N, r) ? N : chirp_length(N);
 }
 
+// threads per pencil of the runtime engine, from the length its stages run
+// at: ceil(L/7) for lengths with a factor 7 (one radix-7 butterfly per
+// thread; every other stage then has at most its usual count)
+inline int rt_threads(int N) {
+  const int L = stage_length(N);
+  return L % 7 == 0 ? (L + 6) / 7 : (L + KW_E - 1) / KW_E;
+}
+
 // wavenumber of ifftshifted index i (kWaveGrid.m:779-797 then ifftshift):
 // (2 pi/d) * (n/N) with n = i for i < ceil(N/2), else i - N
 inline double kvec(int i, int N, double d) {
@@ -166,14 +174,20 @@ inline size_t launch_lds(PassKind k, int fixed, const PassArgs& a, size_t full) 
              : full;
 }
 
-// strided y passes over several buffers give each buffer blocks of its own
-// (KW_YSPLIT=0: one block loops over the buffers)
-inline bool ysplit_on() {
-  static const bool on = [] {
-    const char* e = std::getenv("KW_YSPLIT");
-    return !(e && std::strcmp(e, "0") == 0);
-  }();
-  return on;
+// Buffers of a launch that get blocks of their own (1: a block does them
+// all, one after another).  The strided y passes always split.  x_grad and
+// the last-axis passes of the divergence and the absorbing terms work through
+// independent buffers, so a launch of few threads splits them too: below
+// about four wavefronts per SIMD a block's buffers one after another are its
+// latency, above that the split only repeats its set-up and table reads.
+constexpr int64_t kSplitThreads = 256 * 4 * 64 * 4;
+inline int split_buffers(PassKind k, const PassArgs& a, int dim, int64_t threads) {
+  if (k == PK_YFWD || k == PK_YINV) return a.nbuf;
+  if (threads >= kSplitThreads) return 1;
+  if (k == PK_X_GRAD) return dim;
+  if (k == PK_SPEC && a.mode == SM_DIV) return dim;
+  if (k == PK_SPEC && a.mode == SM_ABS) return 2;
+  return 1;
 }
 
 inline int max_pencils_env() {
@@ -215,6 +229,7 @@ struct Sim {
   ProbDev P{};
   ProbDev* dP = nullptr;
   int32_t* d_tile0 = nullptr;
+  const bool no_fixed = std::getenv("KW_NO_FIXED") != nullptr;  // runtime lengths only
   Tiles tiles;  // pencils per block chosen for this grid (plan_launches)
   void* stream = nullptr;
   bool own_stream = true;
@@ -355,7 +370,7 @@ struct Sim {
 
   // compile-time FFT length of the kernel variant for a pass (0: runtime)
   int fixed_len(PassKind k) const {
-    if (std::getenv("KW_NO_FIXED")) return 0;
+    if (no_fixed) return 0;
     const int N = (k == PK_YFWD || k == PK_YINV) ? G.Ny
                   : (k == PK_SPEC)               ? (G.dim == 3 ? G.Nz : G.Ny)
                                                  : G.Nx;
@@ -370,9 +385,10 @@ struct Sim {
     const int fx = fixed_len(k);
     PassArgs a = a0;
     int nb = g->nb;
-    if ((k == PK_YFWD || k == PK_YINV) && a.nbuf > 1 && ysplit_on()) {
+    const int split = split_buffers(k, a, G.dim, (int64_t)nb * g->T);
+    if (split > 1) {
       a.ysplit = nb;
-      nb *= a.nbuf;
+      nb *= split;
     }
     timed((int)k, timing ? pass_bytes(k, a) : 0.0,
           [&]() { launch_pass(k, fx, G.dim, nb, g->T, launch_lds(k, fx, a, g->lds), B, a, stream); });
@@ -470,13 +486,7 @@ struct Sim {
   void plan_launches() {
     const size_t maxl = dev_max_lds();
     const int capP = max_pencils_env();
-    // threads per pencil of the runtime engine, from the length its stages
-    // run at: ceil(L/7) for lengths with a factor 7 (one radix-7 butterfly
-    // per thread; every other stage then has at most its usual count)
-    auto Gof = [](int N) {
-      const int L = stage_length(N);
-      return L % 7 == 0 ? (L + 6) / 7 : (L + KW_E - 1) / KW_E;
-    };
+    auto Gof = [](int N) { return rt_threads(N); };
     // x pass: <= 256 threads, LDS Nx twiddles + P * kNPX padded pencils; the
     // fixed-length x kernels run x_threads(Nx) threads per pencil
     {
@@ -496,11 +506,14 @@ struct Sim {
       lx.lds = pencil * (size_t)P + twb;
       if (Gx > 512 || lx.lds > maxl) fail(KW_EUNSUP, "grid size Nx too large for the x pass");
     }
+    // (the strided families' tiles also fit the runtime engine's threads per
+    // pencil, which a group of uneven sizes uses: see Group::rebuild)
     // strided y pass (3D): <= 1024 threads, LDS Ny twiddles + P*(Ny+1)
     if (G.dim == 3) {
-      const int Gy = Gof(G.Ny);
+      const int Gy = fixed_len(PK_YFWD) ? strided_threads(G.Ny) : Gof(G.Ny);
       const int Ly = stage_length(G.Ny);
-      int P = std::max(1, std::min(pencils_env("KW_PENCILS_Y", tiles.y ? tiles.y : 16), 1024 / Gy));
+      int P = std::max(1, std::min(pencils_env("KW_PENCILS_Y", tiles.y ? tiles.y : 16),
+                                   1024 / Gof(G.Ny)));
       P = std::min<int64_t>(P, (int64_t)((maxl - sizeof(cf) * Ly) / (sizeof(cf) * (Ly + 1))));
       P = std::max(1, std::min(P, capP));
       this->P.Gy = Gy;
@@ -514,9 +527,10 @@ struct Sim {
     // last-axis pass: <= 1024 threads, LDS N twiddles + 2*P*N
     {
       const int Nl = G.dim == 3 ? G.Nz : G.Ny;
-      const int Gl = Gof(Nl);
+      const int Gl = fixed_len(PK_SPEC) ? strided_threads(Nl) : Gof(Nl);
       const int Ll = stage_length(Nl);
-      int P = std::max(1, std::min(pencils_env("KW_PENCILS_L", tiles.l ? tiles.l : 16), 1024 / Gl));
+      int P = std::max(1, std::min(pencils_env("KW_PENCILS_L", tiles.l ? tiles.l : 16),
+                                   1024 / Gof(Nl)));
       P = std::min<int64_t>(P, (int64_t)((maxl - sizeof(cf) * Ll) / (2 * sizeof(cf) * Ll)));
       P = std::max(1, std::min(P, capP));
       this->P.Gl = Gl;
