@@ -62,6 +62,7 @@ struct XTile {
   // 32-bit offsets of the two rows: first cell (row * Nx), half-spectrum row
   // (row * Wm), Nyquist entry (nspec_main + row); y and z of each row
   uint32_t c0, c1, h0, h1, q0, q1, y0, y1, z0, z1;
+  int32_t s0, s1, s2;  // the sensor points s0 .. s1 - 1 lie in r0, s1 .. s2 - 1 in r1
   LdsPencils lds;
   TwL tw;  // the x twiddles, staged at the start of the block's LDS
 };
@@ -96,6 +97,12 @@ KW_BODY XTile x_tile(Ctx& c, const ProbDev& P, int tile) {
   T.z0 = r0 / (uint32_t)P.Ny;
   T.y1 = r1 % (uint32_t)P.Ny;
   T.z1 = r1 / (uint32_t)P.Ny;
+  T.s0 = T.s1 = T.s2 = 0;
+  if (P.rec_rows) {
+    T.s0 = KW_LD(P.row_sens + T.r0);
+    T.s1 = KW_LD(P.row_sens + T.r0 + 1);
+    T.s2 = KW_LD(P.row_sens + T.r1 + 1);
+  }
   // LDS: the L twiddles of the x transform (put there by x_start), then the
   // pencils (L elements each, padded)
   T.tw = TwL{c.lds()};
@@ -133,6 +140,23 @@ KW_BODY void x_split_store(Ctx& c, const ProbDev& P, const XTile& T, cf* const* 
     }
   }
   c.sync();
+}
+
+// Time series of the sensor points in this pencil's rows, from the values in
+// LDS pencil 0 (real parts: r0, imaginary parts: r1), which the caller has
+// synchronised.  A launch of its own for the same gather took 4 to 5 us of a
+// 35 us step on a 128 x 128 grid, whatever the number of points.
+template <class PC>
+KW_BODY void x_record(PC& c, const ProbDev& P, const XTile& T, float* ts, int t) {
+  if (T.active && t >= P.record_start) {
+    const int64_t col = (int64_t)(t - P.record_start) * P.nsens;
+    for (int k = T.s0 + T.g; k < T.s2; k += T.G) {
+      const bool first = k < T.s1;
+      const cf v = T.lds.get(0, (int)((uint32_t)KW_LD(P.sens_idx + k) - (first ? T.c0 : T.c1)));
+      KW_ST(ts + col + k, first ? v.x : v.y);
+    }
+  }
+  c.sync();  // the transform that follows may write the pencil
 }
 
 // forward transform of NP complex pencils already in LDS, then split/store
@@ -622,15 +646,17 @@ KW_BODY void x_inverse(PC& c, const ProbDev& P, const XTile& T, const cf* S, cf*
 
 // this thread's values (a: row r0, b: row r1) to LDS pencil 0, then the
 // forward x transform of the pencil into the half spectrum S
+// (first writing the record `ts` of the field, when given)
 template <class XS, class PC>
 KW_BODY void x_forward(PC& c, const ProbDev& P, const XTile& T, const float* av, const float* bv,
-                       cf* S) {
+                       cf* S, float* ts = nullptr, int t = 0) {
   KW_PHASE_FENCE();
   if (T.active) {
     auto put = [&](int slot, int n) { T.lds.set(0, n, cf{av[slot], T.has1 ? bv[slot] : 0.f}); };
     XS::last_slots(P.fx, T.g, T.G, T.active, put);
   }
   c.sync();
+  if (ts) x_record(c, P, T, ts, t);
   KW_PHASE_FENCE();
   cf* Sa[1] = {S};
   x_fwd_from_lds<XS, 1>(c, P, T, Sa);
@@ -693,7 +719,8 @@ KW_BODY void body_x_grad(Ctx& cb, const Batch& B, const PassArgs& A) {
       };
       XS::last_slots(P.fx, T.g, T.G, T.active, put);
     }
-    if (!init) x_forward<XS>(c, P, T, av, bv, P.S[d]);
+    if (!init)
+      x_forward<XS>(c, P, T, av, bv, P.S[d], (P.rec_rows & REC_U) ? P.u_ts[d] : nullptr, t);
   }
 }
 
@@ -846,6 +873,7 @@ KW_BODY void x_finish_p(Ctx& c, const ProbDev& P, const XTile& T, cf* pv, int t,
     XS::last_slots(P.fx, T.g, T.G, T.active, fin);
   }
   c.sync();
+  if (P.rec_rows & REC_P) x_record(c, P, T, P.p_ts, t);
 }
 
 // end of the divergence: rho_d update (:912-927), pressure source

@@ -176,6 +176,11 @@ struct ProbDev {
   int32_t p_store_at;
   uint32_t rec_points;
   uint32_t rec_grid;
+  // p and u time series (REC_P, REC_U) that the x passes write themselves,
+  // for binary masks whose points ascend: the points of row r are
+  // row_sens[r] .. row_sens[r + 1] - 1
+  uint32_t rec_rows;
+  const int32_t* row_sens;
   // first step at which the pressure held a non-finite value (0: none),
   // written by the kernels that form p; device memory, or pinned host memory
   // the engine reads after each round without a copy

@@ -635,6 +635,21 @@ std::unique_ptr<Sim> create_sim(const kw_problem* pr_in, void* stream, Arena* ar
       for (int64_t i = 0; i < S->nsens; ++i)
         idx[i] = pr->sensor_mask_index ? (int32_t)(pr->sensor_mask_index[i] - 1) : (int32_t)i;
       P.sens_idx = S->upload(idx);
+      // p and u time series of ascending points are written by the x passes
+      // (the 'WSWS-FFT' record of u swaps its last radial column in after
+      // the step); any other point statistic needs the point kernel, which
+      // then writes them all
+      if (P.rec_points && (P.rec_points & ~(uint32_t)(KW_REC_P | KW_REC_U)) == 0 && !S->as_ws &&
+          std::is_sorted(idx.begin(), idx.end())) {
+        std::vector<int32_t> rows(G.nrows + 1);
+        for (int64_t r = 0, k = 0; r <= G.nrows; ++r) {
+          while (k < S->nsens && (int64_t)idx[k] < r * G.Nx) ++k;
+          rows[r] = (int32_t)k;
+        }
+        P.row_sens = S->upload(rows);
+        P.rec_rows = P.rec_points;
+        P.rec_points = 0;
+      }
     }
     if (directivity && (S->record & KW_REC_P)) {
       // directionalResponse.m: one k-space filter per unique angle, built on
@@ -1042,6 +1057,7 @@ static void record_step(Sim& S, int t, bool init) {
   uint32_t pts = S.record & (kPointP | kPointU);
   if (S.full_mask && !init) pts &= ~kPointP;  // fused into the p producer
   if (S.directivity) pts &= ~(uint32_t)KW_REC_P;  // the directional p below
+  if (!init) pts &= ~S.P.rec_rows;  // written by the x passes
   if (pts) {
     EwArgs e{};
     e.kind = EW_RECORD_POINTS;
