@@ -159,8 +159,15 @@ __device__ __forceinline__ int kw_fresh(int v) {
   __asm__ volatile("" : "+v"(v));
   return v;
 }
+// the same for a uniform constant: keeps the constants of one radix from
+// being held in scalar registers across the code of all others
+__device__ __forceinline__ float kw_fresh_s(float v) {
+  __asm__ volatile("" : "+s"(v));
+  return v;
+}
 #else
 inline int kw_fresh(int v) { return v; }
+inline float kw_fresh_s(float v) { return v; }
 #endif
 
 // Scheduling fence between epilogue phases: each phase batches its own

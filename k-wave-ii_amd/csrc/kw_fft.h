@@ -1,4 +1,4 @@
-// Mixed-radix (2, 3, 4, 5, 8) Stockham FFT over pencils staged in LDS.
+// Mixed-radix Stockham FFT over pencils staged in LDS.
 //
 // A pencil of length N is transformed by G threads.  Stage s with radix R
 // and Ns = product of the radices before it performs N/R butterflies; the
@@ -23,7 +23,7 @@
 // epilogues can keep per-output values in registers across transforms.
 //
 // Two engines share the stage code: `fft_rt` takes a runtime plan (any
-// length that factors into 2, 3 and 5; one code path per radix) and
+// length that factors into 2 .. 13; one code path per radix) and
 // `fft_ct<N>` a length fixed at compile time, for which every index is a
 // constant and the stages unroll into straight-line code.
 //
@@ -38,8 +38,8 @@
 
 namespace kw {
 
-// A transform of length N.  For N = 2^a 3^b 5^c 7^d the stages run at
-// length L = N.  Any other N runs as Bluestein's chirp-z transform: with the
+// A transform of length N.  For N = 2^a 3^b 5^c 7^d 11^e 13^f the stages run
+// at length L = N.  Any other N runs as Bluestein's chirp-z transform: with the
 // chirp w_n = exp(-i pi n^2 / N), X_k = w_k sum_n (x_n w_n) conj(w_(k-n)),
 // a circular convolution of length L >= 2N - 1 (L = 2^a 3^b 5^c) computed
 // with two length-L transforms in LDS; `chirp` (N entries) and `bspec`
@@ -68,9 +68,9 @@ struct CtPlan {
 constexpr int kStageCost = 3;
 
 // elements of one stage of radix R per thread
-constexpr int ct_stage_work(int N, int R, int G) { return (N / R + G - 1) / G * R; }
+KW_HOSTDEV constexpr int ct_stage_work(int N, int R, int G) { return (N / R + G - 1) / G * R; }
 
-constexpr void ct_search(int N, int rest, int G, int emax, CtPlan cur, int cost, int top,
+KW_HOSTDEV constexpr void ct_search(int N, int rest, int G, int emax, CtPlan cur, int cost, int top,
                          CtPlan& best) {
   if (rest == 1) {
     if (cur.nst > 0 && cost < best.cost) {
@@ -92,16 +92,17 @@ constexpr void ct_search(int N, int rest, int G, int emax, CtPlan cur, int cost,
   }
 }
 
-// strided plan of length N with G threads, largest radix first (the first
-// stage has no twiddles)
-constexpr CtPlan ct_strided(int N, int G) {
+// strided plan of length N with G threads, at most 12 elements per thread,
+// largest radix first (the first stage has no twiddles)
+KW_HOSTDEV constexpr CtPlan ct_strided(int N, int G) {
   CtPlan best;
   ct_search(N, N, G, 12, CtPlan{}, 0, 12, best);
   return best;
 }
 // threads per pencil of the strided plan: the least work over all lanes,
-// then the most threads
-constexpr int strided_threads(int N) {
+// then the most threads (half the elements per thread and five stages instead
+// of four took the last axis of 1024 x 1024 from 21 to 23 us)
+KW_HOSTDEV constexpr int strided_threads(int N) {
   int g = 0, work = 1 << 30;
   for (int G = (N + 11) / 12; G <= (N + 7) / 8; ++G) {
     const CtPlan p = ct_strided(N, G);
@@ -114,7 +115,7 @@ constexpr int strided_threads(int N) {
 }
 // x plan: the stage that leaves a thread the fewest elements last, the
 // largest of the others first
-constexpr CtPlan ct_xplan(int N, int G) {
+KW_HOSTDEV constexpr CtPlan ct_xplan(int N, int G) {
   CtPlan p;
   ct_search(N, N, G, 12, CtPlan{}, 0, 10, p);
   int last = 0;
@@ -132,7 +133,8 @@ struct MaxB {
   static constexpr int v = (KW_E + R - 1) / R;
 };
 // lengths with a factor 7 run with G = ceil(N/7) threads (see kw_sim.h), so
-// a radix-7 stage has one butterfly per thread
+// a radix-7 stage has one butterfly per thread, as the larger radices have
+// with any G >= N / 8
 template <>
 struct MaxB<7> {
   static constexpr int v = 1;
@@ -198,6 +200,17 @@ KW_BODY cf fetch(Src& src, int j, int n, int slot) {
     return src(j, n);
 }
 
+// x times a constant held as a rounded float and its remainder.  A radix's
+// rounded sine is wrong by up to 3e-8 in every transform of a simulation, the
+// same way each step: over 400 steps of 600 points the radix-3 and radix-5
+// constants made most of the error against double precision.
+struct Const2 {
+  float hi, lo;
+  constexpr Const2(double v) : hi((float)v), lo((float)(v - (double)(float)v)) {}
+};
+KW_BODY float mulc(float x, const Const2& k) { return x * k.hi + x * k.lo; }
+KW_BODY cf mulc(cf a, const Const2& k) { return cf{mulc(a.x, k), mulc(a.y, k)}; }
+
 // radix-R DFT in place; forward uses exp(-2 pi i rs/R), inverse exp(+...)
 template <int R, bool INV>
 KW_BODY void dft(cf* v);
@@ -215,11 +228,11 @@ KW_BODY void dft<2, true>(cf* v) {
 
 template <bool INV>
 KW_BODY void dft3(cf* v) {
-  const float s3 = 0.866025403784438646763723170752936183f;  // sin(2 pi/3)
+  constexpr Const2 s3(0.866025403784438646763723170752936183);  // sin(2 pi/3)
   cf t = cadd(v[1], v[2]);
   cf d = csub(v[1], v[2]);
   cf m = cf{v[0].x - 0.5f * t.x, v[0].y - 0.5f * t.y};
-  cf sd = cscale(d, s3);
+  cf sd = mulc(d, s3);
   // forward: X1 = m - i sd, X2 = m + i sd
   cf isd = INV ? cmul_pi(sd) : cmul_mi(sd);
   v[0] = cadd(v[0], t);
@@ -251,17 +264,24 @@ KW_BODY void dft<4, true>(cf* v) { dft4<true>(v); }
 
 template <bool INV>
 KW_BODY void dft5(cf* v) {
-  const float c1 = 0.309016994374947424102293417182819059f;   // cos(2 pi/5)
-  const float c2 = -0.809016994374947424102293417182819059f;  // cos(4 pi/5)
-  const float s1 = 0.951056516295153572116439333379382143f;   // sin(2 pi/5)
-  const float s2 = 0.587785252292473129168705954639072769f;   // sin(4 pi/5)
+  constexpr Const2 c1(0.309016994374947424102293417182819059);   // cos(2 pi/5)
+  constexpr Const2 c2(-0.809016994374947424102293417182819059);  // cos(4 pi/5)
+  constexpr Const2 s1(0.951056516295153572116439333379382143);   // sin(2 pi/5)
+  constexpr Const2 s2(0.587785252292473129168705954639072769);   // sin(4 pi/5)
   cf a1 = cadd(v[1], v[4]), b1 = csub(v[1], v[4]);
   cf a2 = cadd(v[2], v[3]), b2 = csub(v[2], v[3]);
   cf x0 = v[0];
-  cf m1 = cf{x0.x + c1 * a1.x + c2 * a2.x, x0.y + c1 * a1.y + c2 * a2.y};
-  cf m2 = cf{x0.x + c2 * a1.x + c1 * a2.x, x0.y + c2 * a1.y + c1 * a2.y};
-  cf n1 = cf{s1 * b1.x + s2 * b2.x, s1 * b1.y + s2 * b2.y};
-  cf n2 = cf{s2 * b1.x - s1 * b2.x, s2 * b1.y - s1 * b2.y};
+  // z + p a + q b, the remainders of the constants first
+  auto lin = [](float z, const Const2& p, float a, const Const2& q, float b) {
+    return ((z + (p.lo * a + q.lo * b)) + p.hi * a) + q.hi * b;
+  };
+  auto dif = [](const Const2& p, float a, const Const2& q, float b) {
+    return ((p.lo * a - q.lo * b) + p.hi * a) - q.hi * b;
+  };
+  cf m1 = cf{lin(x0.x, c1, a1.x, c2, a2.x), lin(x0.y, c1, a1.y, c2, a2.y)};
+  cf m2 = cf{lin(x0.x, c2, a1.x, c1, a2.x), lin(x0.y, c2, a1.y, c1, a2.y)};
+  cf n1 = cf{lin(0.f, s1, b1.x, s2, b2.x), lin(0.f, s1, b1.y, s2, b2.y)};
+  cf n2 = cf{dif(s2, b1.x, s1, b2.x), dif(s2, b1.y, s1, b2.y)};
   // forward: X1 = m1 - i n1, X4 = m1 + i n1, X2 = m2 - i n2, X3 = m2 + i n2
   cf in1 = INV ? cmul_pi(n1) : cmul_mi(n1);
   cf in2 = INV ? cmul_pi(n2) : cmul_mi(n2);
@@ -276,56 +296,86 @@ KW_BODY void dft<5, false>(cf* v) { dft5<false>(v); }
 template <>
 KW_BODY void dft<5, true>(cf* v) { dft5<true>(v); }
 
-// radix 7 from the pairs a_k = v_k + v_(7-k), b_k = v_k - v_(7-k):
-// X_j = v_0 + sum_k cos(2 pi jk/7) a_k -+ i sum_k sin(2 pi jk/7) b_k
-template <bool INV>
-KW_BODY void dft7(cf* v) {
-  const float c1 = 0.6234898018587336f, c2 = -0.22252093395631434f, c3 = -0.9009688679024191f;
-  const float s1 = 0.7818314824680298f, s2 = 0.9749279121818236f, s3 = 0.43388373911755823f;
-  const cf a1 = cadd(v[1], v[6]), b1 = csub(v[1], v[6]);
-  const cf a2 = cadd(v[2], v[5]), b2 = csub(v[2], v[5]);
-  const cf a3 = cadd(v[3], v[4]), b3 = csub(v[3], v[4]);
+// odd prime radix from the pairs a_k = v_k + v_(R-k), b_k = v_k - v_(R-k):
+// X_j = v_0 + sum_k cos(2 pi jk/R) a_k -+ i sum_k sin(2 pi jk/R) b_k
+template <int R>
+struct PrimeTrig;  // cos and sin of 2 pi m / R, m = 1 .. (R - 1) / 2
+template <>
+struct PrimeTrig<7> {
+  static constexpr float c[3] = {0.6234898018587335f, -0.2225209339563144f, -0.9009688679024191f};
+  static constexpr float s[3] = {0.7818314824680298f, 0.9749279121818236f, 0.4338837391175581f};
+};
+template <>
+struct PrimeTrig<11> {
+  static constexpr float c[5] = {0.8412535328311812f, 0.4154150130018864f, -0.142314838273285f,
+                                 -0.654860733945285f, -0.9594929736144974f};
+  static constexpr float s[5] = {0.5406408174555976f, 0.9096319953545184f, 0.9898214418809327f,
+                                 0.7557495743542583f, 0.2817325568414297f};
+};
+template <>
+struct PrimeTrig<13> {
+  static constexpr float c[6] = {0.8854560256532099f, 0.5680647467311558f, 0.1205366802553230f,
+                                 -0.3546048870425356f, -0.7485107481711011f, -0.9709418174260521f};
+  static constexpr float s[6] = {0.4647231720437685f, 0.8229838658936564f, 0.9927088740980540f,
+                                 0.9350162426854148f, 0.6631226582407952f, 0.2393156642875578f};
+};
+template <int R, bool INV>
+KW_BODY void dft_prime(cf* v) {
+  constexpr int H = (R - 1) / 2;
+  cf a[H], b[H];
+#pragma unroll
+  for (int k = 0; k < H; ++k) {
+    a[k] = cadd(v[k + 1], v[R - 1 - k]);
+    b[k] = csub(v[k + 1], v[R - 1 - k]);
+  }
+  float co_[H], si_[H];
+#pragma unroll
+  for (int k = 0; k < H; ++k) {
+    co_[k] = kw_fresh_s(PrimeTrig<R>::c[k]);
+    si_[k] = kw_fresh_s(PrimeTrig<R>::s[k]);
+  }
   const cf x0 = v[0];
-  auto lin = [](cf z, float p, cf a, float q, cf b, float r, cf c) {
-    return cf{z.x + p * a.x + q * b.x + r * c.x, z.y + p * a.y + q * b.y + r * c.y};
-  };
-  const cf zero{0.f, 0.f};
-  const cf m1 = lin(x0, c1, a1, c2, a2, c3, a3);
-  const cf m2 = lin(x0, c2, a1, c3, a2, c1, a3);
-  const cf m3 = lin(x0, c3, a1, c1, a2, c2, a3);
-  const cf n1 = lin(zero, s1, b1, s2, b2, s3, b3);
-  const cf n2 = lin(zero, s2, b1, -s3, b2, -s1, b3);
-  const cf n3 = lin(zero, s3, b1, -s1, b2, s2, b3);
-  // forward: X_j = m_j - i n_j, X_(7-j) = m_j + i n_j
-  const cf i1 = INV ? cmul_pi(n1) : cmul_mi(n1);
-  const cf i2 = INV ? cmul_pi(n2) : cmul_mi(n2);
-  const cf i3 = INV ? cmul_pi(n3) : cmul_mi(n3);
-  v[0] = cf{x0.x + a1.x + a2.x + a3.x, x0.y + a1.y + a2.y + a3.y};
-  v[1] = cadd(m1, i1);
-  v[6] = csub(m1, i1);
-  v[2] = cadd(m2, i2);
-  v[5] = csub(m2, i2);
-  v[3] = cadd(m3, i3);
-  v[4] = csub(m3, i3);
+  cf sum = x0;
+#pragma unroll
+  for (int k = 0; k < H; ++k) sum = cadd(sum, a[k]);
+  v[0] = sum;
+#pragma unroll
+  for (int j = 1; j <= H; ++j) {
+    cf m = x0, n = cf{0.f, 0.f};
+#pragma unroll
+    for (int k = 1; k <= H; ++k) {
+      const int q = j * k % R;
+      const float co = co_[(q <= H ? q : R - q) - 1];
+      const float si = q <= H ? si_[q - 1] : -si_[R - q - 1];
+      m = cf{m.x + co * a[k - 1].x, m.y + co * a[k - 1].y};
+      n = cf{n.x + si * b[k - 1].x, n.y + si * b[k - 1].y};
+    }
+    // forward: X_j = m - i n, X_(R-j) = m + i n
+    const cf in = INV ? cmul_pi(n) : cmul_mi(n);
+    v[j] = cadd(m, in);
+    v[R - j] = csub(m, in);
+  }
 }
-template <>
-KW_BODY void dft<7, false>(cf* v) { dft7<false>(v); }
-template <>
-KW_BODY void dft<7, true>(cf* v) { dft7<true>(v); }
+template <> KW_BODY void dft<7, false>(cf* v) { dft_prime<7, false>(v); }
+template <> KW_BODY void dft<7, true>(cf* v) { dft_prime<7, true>(v); }
+template <> KW_BODY void dft<11, false>(cf* v) { dft_prime<11, false>(v); }
+template <> KW_BODY void dft<11, true>(cf* v) { dft_prime<11, true>(v); }
+template <> KW_BODY void dft<13, false>(cf* v) { dft_prime<13, false>(v); }
+template <> KW_BODY void dft<13, true>(cf* v) { dft_prime<13, true>(v); }
 
 template <bool INV>
 KW_BODY void dft8(cf* v) {
-  const float h = 0.707106781186547524400844362104849039f;
+  constexpr Const2 h(0.707106781186547524400844362104849039);
   cf e[4] = {v[0], v[2], v[4], v[6]};
   cf o[4] = {v[1], v[3], v[5], v[7]};
   dft4<INV>(e);
   dft4<INV>(o);
   // o[k] *= w8^k, w8 = exp(-+ 2 pi i/8)
-  cf w1 = INV ? cf{h, h} : cf{h, -h};
-  cf w3 = INV ? cf{-h, h} : cf{-h, -h};
-  o[1] = cmul(o[1], w1);
+  const cf a = mulc(cf{o[1].x - o[1].y, o[1].x + o[1].y}, h);  // o[1] exp(+i pi/4)
+  const cf b = mulc(cf{o[3].x - o[3].y, o[3].x + o[3].y}, h);  // o[3] exp(+i pi/4)
+  o[1] = INV ? a : cf{a.y, -a.x};
   o[2] = INV ? cmul_pi(o[2]) : cmul_mi(o[2]);
-  o[3] = cmul(o[3], w3);
+  o[3] = INV ? cmul_pi(b) : cf{-b.x, -b.y};
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
     v[k] = cadd(e[k], o[k]);
@@ -370,8 +420,9 @@ template <> KW_BODY void dft<12, true>(cf* v) { dft_pfa<3, 4, true>(v); }
 
 // multiply by exp(-+ i angle) given its cosine and sine
 template <bool INV>
-KW_BODY cf cturn(cf a, float co, float si) {
-  return INV ? cmul(a, cf{co, si}) : cmul(a, cf{co, -si});
+KW_BODY cf cturn(cf a, const Const2& co, const Const2& si) {
+  const cf p = mulc(a, co), q = mulc(a, si);
+  return INV ? cf{p.x - q.y, p.y + q.x} : cf{p.x + q.y, p.y - q.x};
 }
 
 // radix 9 as 3 x 3: input 3 n1 + n2, output k1 + 3 k2, constant twiddles
@@ -379,9 +430,9 @@ KW_BODY cf cturn(cf a, float co, float si) {
 template <bool INV>
 KW_BODY void dft9(cf* v) {
   // cos and sin of 2 pi j / 9, j = 1, 2, 4
-  const float c1 = 0.766044443118978f, s1 = 0.6427876096865393f;
-  const float c2 = 0.17364817766693036f, s2 = 0.984807753012208f;
-  const float c4 = -0.9396926207859084f, s4 = 0.3420201433256687f;
+  constexpr Const2 c1(0.766044443118978035202392650555416673), s1(0.642787609686539326322643409907263432);
+  constexpr Const2 c2(0.173648177666930348851716626769314796), s2(0.984807753012208059366743024589523013);
+  constexpr Const2 c4(-0.939692620785908384054109277324731469), s4(0.342020143325668733044099614682259580);
   cf t[3][3];
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
@@ -414,9 +465,15 @@ KW_BODY int mod_ns(int b, int Ns) {
 // number of butterflies per thread (exact for the fixed-length engine, an
 // upper bound for the runtime engine).  `src` must be safe to call for
 // every thread, including threads with active == false.
+// `rns` is 1 / Ns for a runtime Ns (b mod Ns by an integer division would be
+// some forty instructions per butterfly; in float it is exact for b + 0.5
+// below 2^20) and 0 for a compile-time one.
 template <int R, int NP, bool INV, int MB, class Ctx, class TW, class Src, class Dst>
 KW_BODY void stage(Ctx& c, int N, int Ns, int G, int g, bool active, const TW& tw, Src& src,
-                   Dst& dst) {
+                   Dst& dst, float rns = 0.f) {
+  auto mod = [&](int b) {
+    return rns != 0.f ? b - Ns * (int)(((float)b + 0.5f) * rns) : mod_ns(b, Ns);
+  };
   const int nb = N / R;
   const int twstep = N / (Ns * R);
   cf v[NP][MB][R];
@@ -429,7 +486,7 @@ KW_BODY void stage(Ctx& c, int N, int Ns, int G, int g, bool active, const TW& t
     if (MB * G == nb || b < nb) {
       cf w[R];
       if (Ns > 1) {
-        const int k = mod_ns(b, Ns);
+        const int k = mod(b);
 #pragma unroll
         for (int r = 1; r < R; ++r) w[r] = twiddle<INV>(tw, k * r * twstep);
       }
@@ -455,7 +512,7 @@ KW_BODY void stage(Ctx& c, int N, int Ns, int G, int g, bool active, const TW& t
     for (int m = 0; m < MB; ++m) {
       const int b = g + m * G;
       if (active && (MB * G == nb || b < nb)) {
-        const int k = mod_ns(b, Ns);
+        const int k = mod(b);
         const int j0 = (b - k) * R + k;
 #pragma unroll
         for (int r = 0; r < R; ++r) dst(j, j0 + r * Ns, v[j][m][r], m * R + r);
@@ -478,7 +535,7 @@ struct LdsPencils {
 };
 
 // ---- runtime-length engine --------------------------------------------------
-// Any N = 2^a 3^b 5^c 7^d.  The transform is staged entirely in LDS: a strided,
+// Any N = 2^a 3^b 5^c 7^d 11^e 13^f.  The transform is staged entirely in LDS: a strided,
 // coalesced pass loads the pencil into LDS through the caller's functor, the
 // Stockham stages run from LDS to LDS, and a strided pass hands element
 // n = g + i*G to the caller as slot i.  The caller's functors are
@@ -500,14 +557,25 @@ KW_BODY void fft_stages_rt(Ctx& c, const FftPlan& pl, const TW& tw, int g, int G
   const int L = pl.L;
   for (int s = 0; s < pl.nst; ++s) {
     const int R = pl.radix[s];
+    const float rns = 1.0f / (float)Ns;
+    // a fresh thread index per stage, or every radix's element indices are
+    // hoisted out of this loop and spill
+    const int gs = kw_fresh(g);
+#define KW_RT_STAGE(RR)                                                                           \
+  case RR: stage<RR, NP, INV, MaxB<RR>::v>(c, L, Ns, G, gs, active, tw, lsrc, ldst, rns); break;
     switch (R) {
-      case 2: stage<2, NP, INV, MaxB<2>::v>(c, L, Ns, G, g, active, tw, lsrc, ldst); break;
-      case 3: stage<3, NP, INV, MaxB<3>::v>(c, L, Ns, G, g, active, tw, lsrc, ldst); break;
-      case 4: stage<4, NP, INV, MaxB<4>::v>(c, L, Ns, G, g, active, tw, lsrc, ldst); break;
-      case 5: stage<5, NP, INV, MaxB<5>::v>(c, L, Ns, G, g, active, tw, lsrc, ldst); break;
-      case 7: stage<7, NP, INV, MaxB<7>::v>(c, L, Ns, G, g, active, tw, lsrc, ldst); break;
-      default: stage<8, NP, INV, MaxB<8>::v>(c, L, Ns, G, g, active, tw, lsrc, ldst); break;
+      KW_RT_STAGE(2)
+      KW_RT_STAGE(3)
+      KW_RT_STAGE(4)
+      KW_RT_STAGE(5)
+      KW_RT_STAGE(7)
+      KW_RT_STAGE(8)
+      KW_RT_STAGE(9)
+      KW_RT_STAGE(10)
+      KW_RT_STAGE(11)
+      KW_RT_STAGE(13)
     }
+#undef KW_RT_STAGE
     Ns *= R;
   }
 }
@@ -754,11 +822,26 @@ KW_HOSTDEV constexpr int ct_threads(int N) { return (N + KW_E - 1) / KW_E; }
 // that leaves a thread at most six elements, so that every pencil lies in one
 // wavefront and the stages synchronise with wavefront barriers instead of
 // block barriers (the extra lanes idle in stages with fewer butterflies than
-// lanes); lengths above 384 take ceil(N / KW_E)
+// lanes); lengths above 384 take a wavefront per 256 elements (one step of 600
+// points 37 -> 29 us against ceil(N / KW_E))
 KW_HOSTDEV constexpr int x_threads(int N) {
   for (int p = 1; p <= 64; p <<= 1)
     if (6 * p >= N) return p;
-  return ct_threads(N) <= 64 ? 64 : ct_threads(N);
+  return (N + 255) / 256 * 64;
+}
+
+// elements a thread owns after an x transform, and whether the 3-D x_div
+// kernel of that length also writes the p time series: it holds a dozen
+// registers per element, and from six elements on the record's few more cost
+// it a wavefront per SIMD (192: 128 -> 129 VGPRs, 74 -> 90 us at 192^3; at
+// 128^3 and 144 x 160 x 192 no difference).  2-D grids always record.
+KW_HOSTDEV constexpr int x_slots(int N) {
+  const int G = x_threads(N);
+  const CtPlan p = ct_xplan(N, G);
+  return ct_stage_work(N, p.r[p.nst - 1], G);
+}
+KW_HOSTDEV constexpr bool x_div_records(int dim, int fixed) {
+  return dim == 2 || fixed == 0 || x_slots(fixed) < 6;
 }
 
 template <class Sh>

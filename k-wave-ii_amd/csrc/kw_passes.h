@@ -62,7 +62,6 @@ struct XTile {
   // 32-bit offsets of the two rows: first cell (row * Nx), half-spectrum row
   // (row * Wm), Nyquist entry (nspec_main + row); y and z of each row
   uint32_t c0, c1, h0, h1, q0, q1, y0, y1, z0, z1;
-  int32_t s0, s1, s2;  // the sensor points s0 .. s1 - 1 lie in r0, s1 .. s2 - 1 in r1
   LdsPencils lds;
   TwL tw;  // the x twiddles, staged at the start of the block's LDS
 };
@@ -97,12 +96,6 @@ KW_BODY XTile x_tile(Ctx& c, const ProbDev& P, int tile) {
   T.z0 = r0 / (uint32_t)P.Ny;
   T.y1 = r1 % (uint32_t)P.Ny;
   T.z1 = r1 / (uint32_t)P.Ny;
-  T.s0 = T.s1 = T.s2 = 0;
-  if (P.rec_rows) {
-    T.s0 = KW_LD(P.row_sens + T.r0);
-    T.s1 = KW_LD(P.row_sens + T.r0 + 1);
-    T.s2 = KW_LD(P.row_sens + T.r1 + 1);
-  }
   // LDS: the L twiddles of the x transform (put there by x_start), then the
   // pencils (L elements each, padded)
   T.tw = TwL{c.lds()};
@@ -150,8 +143,13 @@ template <class PC>
 KW_BODY void x_record(PC& c, const ProbDev& P, const XTile& T, float* ts, int t) {
   if (T.active && t >= P.record_start) {
     const int64_t col = (int64_t)(t - P.record_start) * P.nsens;
-    for (int k = T.s0 + T.g; k < T.s2; k += T.G) {
-      const bool first = k < T.s1;
+    // points s0 .. s1 - 1 lie in r0, s1 .. s2 - 1 in r1 (read here: held from
+    // the block's start they cost x_div registers it has not got, 74 -> 92 us
+    // at 192^3)
+    const int s0 = KW_LD(P.row_sens + T.r0), s1 = KW_LD(P.row_sens + T.r0 + 1);
+    const int s2 = KW_LD(P.row_sens + T.r1 + 1);
+    for (int k = s0 + T.g; k < s2; k += T.G) {
+      const bool first = k < s1;
       const cf v = T.lds.get(0, (int)((uint32_t)KW_LD(P.sens_idx + k) - (first ? T.c0 : T.c1)));
       KW_ST(ts + col + k, first ? v.x : v.y);
     }
@@ -767,7 +765,8 @@ KW_BODY float tr_rho(const ProbDev& P, float p, float c2) {
 // New p of the cells of this thread's slots (pv[slot] = rows r0, r1): time
 // reversal, sensors and the optional store, each as one batched phase over
 // the slots; finally the values go to LDS pencil 0 for fft_x(p).
-template <class XS, class Ctx>
+// (REC: and its time series, when P.rec_rows asks for it)
+template <class XS, bool REC, class Ctx>
 KW_BODY void x_finish_p(Ctx& c, const ProbDev& P, const XTile& T, cf* pv, int t, bool store) {
   const int N = P.Nx;
   {
@@ -873,7 +872,9 @@ KW_BODY void x_finish_p(Ctx& c, const ProbDev& P, const XTile& T, cf* pv, int t,
     XS::last_slots(P.fx, T.g, T.G, T.active, fin);
   }
   c.sync();
-  if (P.rec_rows & REC_P) x_record(c, P, T, P.p_ts, t);
+  if constexpr (REC) {
+    if (P.rec_rows & REC_P) x_record(c, P, T, P.p_ts, t);
+  }
 }
 
 // end of the divergence: rho_d update (:912-927), pressure source
@@ -1004,7 +1005,7 @@ KW_BODY void body_x_div(Ctx& cb, const Batch& B, const PassArgs& A) {
       };
       XS::last_slots(P.fx, T.g, T.G, T.active, f);
     });
-    x_finish_p<XS>(c, P, T, pv, t, store_p);
+    x_finish_p<XS, x_div_records(DIM, XS::fixed)>(c, P, T, pv, t, store_p);
     cf* S0[1] = {P.S[0]};
     x_fwd_from_lds<XS, 1>(c, P, T, S0);
   }
@@ -1061,7 +1062,7 @@ KW_BODY void body_x_eos(Ctx& cb, const Batch& B, const PassArgs& A) {
     };
     XS::last_slots(P.fx, T.g, T.G, T.active, f);
   });
-  x_finish_p<XS>(c, P, T, pv, t, store_p);
+  x_finish_p<XS, true>(c, P, T, pv, t, store_p);
   cf* S0[1] = {P.S[0]};
   x_fwd_from_lds<XS, 1>(c, P, T, S0);
 }

@@ -103,6 +103,19 @@ static float* source_km(Sim& S, const kw_time_source& src) {
   return km;
 }
 
+// The step's scalar factors are rounded to single (dt, and c0, rho0 and
+// 1 / rho0 where they are uniform), the same way in every step: up to 2e-7 in
+// the squared speed of every wave, most of the error of a long run in a
+// uniform medium.  A gradient and a divergence carry the square of kappa per
+// step, so kappa takes the square root of what their product lost.
+static double rounding_of(const kw_problem& pr, double dt) {
+  auto lost = [](double v) { return v / (double)(float)v; };
+  double f = lost(dt) * lost(dt);
+  if (!pr.c0) f *= lost(pr.c0_scalar) * lost(pr.c0_scalar);
+  if (!pr.rho0) f *= lost(pr.rho0_scalar) * lost(1.0 / pr.rho0_scalar);
+  return std::sqrt(f);
+}
+
 std::unique_ptr<Sim> create_sim(const kw_problem* pr_in, void* stream, Arena* arena) {
   if (!pr_in) fail(KW_EINVAL, "problem is NULL");
   const int pdim = pr_in->dim;
@@ -495,15 +508,16 @@ std::unique_ptr<Sim> create_sim(const kw_problem* pr_in, void* stream, Arena* ar
     }
     return std::sqrt(acc);
   };
+  const double fit = rounding_of(*pr, dt);
   P.kappa = S->spectral_table([&](int ix, int iy, int iz) {
-    return (use_k ? sinc(cref * kmag(ix, iy, iz) * dt / 2) : 1.0) / Ntot;
+    return (use_k ? sinc(cref * kmag(ix, iy, iz) * dt / 2) : 1.0) * fit / Ntot;
   });
   if (S->axisym) {
     // the radial divergence adds shift_y^- κ fft(u_y / r) (kspaceFirstOrderAS.m:
     // 954-969): κ times the y shift (which carries the 1/(Nx Ny) of the
     // round trip) in one last-axis pass
     S->as_kappa = S->spectral_table([&](int ix, int iy, int iz) {
-      return use_k ? sinc(cref * kmag(ix, iy, iz) * dt / 2) : 1.0;
+      return (use_k ? sinc(cref * kmag(ix, iy, iz) * dt / 2) : 1.0) * fit;
     });
     // ir: + on the copies that hold u_r, - on the mirrored ones, so that
     // ir .* u_r has the even layout of u_r / r (:966-977)
@@ -636,10 +650,13 @@ std::unique_ptr<Sim> create_sim(const kw_problem* pr_in, void* stream, Arena* ar
         idx[i] = pr->sensor_mask_index ? (int32_t)(pr->sensor_mask_index[i] - 1) : (int32_t)i;
       P.sens_idx = S->upload(idx);
       // p and u time series of ascending points are written by the x passes
-      // (the 'WSWS-FFT' record of u swaps its last radial column in after
-      // the step); any other point statistic needs the point kernel, which
-      // then writes them all
-      if (P.rec_points && (P.rec_points & ~(uint32_t)(KW_REC_P | KW_REC_U)) == 0 && !S->as_ws &&
+      // (p by x_eos, or by the x_div kernels that do; the 'WSWS-FFT' record of
+      // u swaps its last radial column in after the step); any other point
+      // statistic needs the point kernel, which then writes them all
+      uint32_t by_rows = KW_REC_U;
+      if (P.eos == EOS_ABSORBING || x_div_records(G.dim, S->fixed_len(PK_X_DIV)))
+        by_rows |= KW_REC_P;
+      if (P.rec_points && (P.rec_points & ~by_rows) == 0 && !S->as_ws &&
           std::is_sorted(idx.begin(), idx.end())) {
         std::vector<int32_t> rows(G.nrows + 1);
         for (int64_t r = 0, k = 0; r <= G.nrows; ++r) {

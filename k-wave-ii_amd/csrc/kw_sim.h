@@ -28,43 +28,52 @@ constexpr double kPi = 3.14159265358979323846264338327950288;
 // operators (double precision)
 // ---------------------------------------------------------------------------
 
-// radices for a length: 8s first, then 4 or 2, then 3s and 5s
+// Radices of the runtime engine for a length, largest first: the sequence
+// with the least ceil(butterflies / G) R + 4 over its stages, the 4 for the
+// LDS round trip and barrier of a stage.  G is the engine's threads per
+// pencil (rt_threads).
+inline void radix_search(int N, int rest, int G, int top, std::vector<int>& cur, int cost,
+                         std::vector<int>& best, int& best_cost) {
+  if (rest == 1) {
+    if (cost < best_cost) {
+      best = cur;
+      best_cost = cost;
+    }
+    return;
+  }
+  if ((int)cur.size() >= KW_MAX_STAGES) return;
+  for (int R : {13, 11, 10, 9, 8, 7, 5, 4, 3, 2}) {
+    if (R > top || rest % R != 0) continue;
+    const int c = cost + (N / R + G - 1) / G * R + 4;
+    if (c >= best_cost) continue;
+    cur.push_back(R);
+    radix_search(N, rest / R, G, R, cur, c, best, best_cost);
+    cur.pop_back();
+  }
+}
+
+// threads per pencil of the runtime engine at stage length L: ceil(L/7) for
+// lengths with a factor 7 (one radix-7 butterfly per thread; every other
+// stage then has at most its usual count)
+inline int stage_threads(int L) { return L % 7 == 0 ? (L + 6) / 7 : (L + KW_E - 1) / KW_E; }
+
 inline bool factorise(int N, std::vector<int>& r) {
   r.clear();
   int n = N;
-  while (n % 8 == 0) {
-    r.push_back(8);
-    n /= 8;
-  }
-  if (n % 4 == 0) {
-    r.push_back(4);
-    n /= 4;
-  }
-  if (n % 2 == 0) {
-    r.push_back(2);
-    n /= 2;
-  }
-  while (n % 3 == 0) {
-    r.push_back(3);
-    n /= 3;
-  }
-  while (n % 5 == 0) {
-    r.push_back(5);
-    n /= 5;
-  }
-  // radix 7 in the runtime engine only (pencils of such lengths run with
-  // G = ceil(N/7) threads: one radix-7 butterfly each)
-  while (n % 7 == 0) {
-    r.push_back(7);
-    n /= 7;
-  }
+  for (int p : {2, 3, 5, 7, 11, 13})
+    while (n % p == 0) n /= p;
+  if (n != 1) return false;
   // N = 1 (the y axis of a 1-D problem): no stages, the transform is the
   // identity
-  return n == 1 && (N == 1 || !r.empty()) && (int)r.size() <= KW_MAX_STAGES;
+  if (N == 1) return true;
+  std::vector<int> cur;
+  int cost = 1 << 30;
+  radix_search(N, N, stage_threads(N), 13, cur, 0, r, cost);
+  return !r.empty();
 }
 
-// length of the chirp-z convolution for a transform of length N that does
-// not factor into 2, 3, 5 and 7: the smallest 2^a 3^b 5^c >= 2N - 1
+// length of the chirp-z convolution for a transform of length N that has a
+// prime factor above 13: the smallest 2^a 3^b 5^c >= 2N - 1
 inline int chirp_length(int N) {
   for (int L = std::max(1, 2 * N - 1);; ++L) {
     int m = L;
@@ -80,13 +89,8 @@ inline int stage_length(int N) {
   return factorise(N, r) ? N : chirp_length(N);
 }
 
-// threads per pencil of the runtime engine, from the length its stages run
-// at: ceil(L/7) for lengths with a factor 7 (one radix-7 butterfly per
-// thread; every other stage then has at most its usual count)
-inline int rt_threads(int N) {
-  const int L = stage_length(N);
-  return L % 7 == 0 ? (L + 6) / 7 : (L + KW_E - 1) / KW_E;
-}
+// threads per pencil of the runtime engine, from the length its stages run at
+inline int rt_threads(int N) { return stage_threads(stage_length(N)); }
 
 // wavenumber of ifftshifted index i (kWaveGrid.m:779-797 then ifftshift):
 // (2 pi/d) * (n/N) with n = i for i < ceil(N/2), else i - N
@@ -107,6 +111,29 @@ inline std::vector<double> pml_profile(int N, double d, double dt, double c, int
     v[N - size + x - 1] = std::exp(-right * dt / 2.0);
   }
   return v;
+}
+
+// exp(-i a) in single precision: of the neighbours of the rounded cosine and
+// sine, the pair whose magnitude is nearest 1, a tenth of the angle's error
+// added.  A step's transforms come in pairs, forward and inverse, whose
+// angles cancel while magnitudes accumulate over the steps.
+inline cf root_of_unity(double a) {
+  const double c = std::cos(a), s = -std::sin(a);
+  cf best{(float)c, (float)s};
+  if (best.x == 0.f || best.y == 0.f || std::fabs(c) < 1e-7 || std::fabs(s) < 1e-7) return best;
+  double least = 1e9;
+  for (int i = -1; i <= 1; ++i)
+    for (int j = -1; j <= 1; ++j) {
+      const float x = i == 0 ? (float)c : std::nextafter((float)c, i * 2.f);
+      const float y = j == 0 ? (float)s : std::nextafter((float)s, j * 2.f);
+      const double m = ((double)x * x + (double)y * y - 1.0) / 2, t = (double)y * c - (double)x * s;
+      const double e = std::fabs(m) + 0.1 * std::fabs(t);
+      if (e < least) {
+        least = e;
+        best = cf{x, y};
+      }
+    }
+  return best;
 }
 
 inline double sinc(double x) { return x == 0.0 ? 1.0 : std::sin(x) / x; }
@@ -490,7 +517,14 @@ struct Sim {
     // x pass: <= 256 threads, LDS Nx twiddles + P * kNPX padded pencils; the
     // fixed-length x kernels run x_threads(Nx) threads per pencil
     {
-      const int Gx = fixed_len(PK_X_GRAD) ? x_threads(G.Nx) : Gof(G.Nx);
+      // (a power of two up to 64 keeps every pencil in one wavefront, whose
+      // barriers cost less than the idle lanes)
+      int Gx = fixed_len(PK_X_GRAD) ? x_threads(G.Nx) : Gof(G.Nx);
+      for (int p = 1; p <= 64 && Gx <= 64; p <<= 1)
+        if (p >= Gx) {
+          Gx = p;
+          break;
+        }
       const int Lx = stage_length(G.Nx);
       const size_t pencil = sizeof(cf) * (size_t)kNPX * x_lds_stride(Lx);
       const size_t twb = sizeof(cf) * (size_t)Lx;
@@ -513,7 +547,7 @@ struct Sim {
       const int Gy = fixed_len(PK_YFWD) ? strided_threads(G.Ny) : Gof(G.Ny);
       const int Ly = stage_length(G.Ny);
       int P = std::max(1, std::min(pencils_env("KW_PENCILS_Y", tiles.y ? tiles.y : 16),
-                                   1024 / Gof(G.Ny)));
+                                   1024 / std::max(Gy, Gof(G.Ny))));
       P = std::min<int64_t>(P, (int64_t)((maxl - sizeof(cf) * Ly) / (sizeof(cf) * (Ly + 1))));
       P = std::max(1, std::min(P, capP));
       this->P.Gy = Gy;
@@ -530,7 +564,7 @@ struct Sim {
       const int Gl = fixed_len(PK_SPEC) ? strided_threads(Nl) : Gof(Nl);
       const int Ll = stage_length(Nl);
       int P = std::max(1, std::min(pencils_env("KW_PENCILS_L", tiles.l ? tiles.l : 16),
-                                   1024 / Gof(Nl)));
+                                   1024 / std::max(Gl, Gof(Nl))));
       P = std::min<int64_t>(P, (int64_t)((maxl - sizeof(cf) * Ll) / (2 * sizeof(cf) * Ll)));
       P = std::max(1, std::min(P, capP));
       this->P.Gl = Gl;
@@ -547,7 +581,7 @@ struct Sim {
   }
 
   // FFT plan of an axis of length N: stages of the radices of N, or for N
-  // with a prime factor above 7 Bluestein's chirp-z transform (kw_fft.h),
+  // with a prime factor above 13 Bluestein's chirp-z transform (kw_fft.h),
   // whose chirp and filter transform are computed here in double precision
   // and rounded once
   FftPlan make_plan(int N) {
@@ -562,8 +596,7 @@ struct Sim {
     for (size_t i = 0; i < r.size(); ++i) pl.radix[i] = r[i];
     std::vector<cf> tw(L);
     for (int j = 0; j < L; ++j) {
-      const double a = 2.0 * kPi * (double)j / (double)L;
-      tw[j] = cf{(float)std::cos(a), (float)-std::sin(a)};
+      tw[j] = root_of_unity(2.0 * kPi * (double)j / (double)L);
     }
     pl.tw = upload(tw);
     if (!direct) {
