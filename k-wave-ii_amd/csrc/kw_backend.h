@@ -7,6 +7,7 @@
 #include <string>
 
 #include "kw_passes.h"
+#include "kw_setup.h"
 
 namespace kw {
 
@@ -39,12 +40,14 @@ int fixed_variant(int N, PassKind kind);
 void launch_pass(PassKind kind, int fixed, int dim, int nblocks, int threads, size_t lds_bytes,
                  const Batch& B, const PassArgs& A, void* stream);
 void launch_ew(int nblocks, const Batch& B, const EwArgs& A, void* stream);
+void launch_setup(const SetupArgs& A, void* stream);
 
 // event timing (GPU only; the emulator returns wall-clock times)
 void* dev_event_create();
 void dev_event_destroy(void* e);
 void dev_event_record(void* e, void* stream);
 double dev_event_elapsed_ms(void* a, void* b);  // synchronises on b
+void dev_event_wait(void* e);                   // until the work before e has finished
 bool dev_event_done(void* e);                   // the work before e has finished
 
 // Graphs of launches: capture what one host thread launches on `stream`

@@ -376,12 +376,18 @@ void launch_ew(int nblocks, const Batch& B, const EwArgs& A, void*) {
   emu_launch(nblocks, EW_T, 0, f);
 }
 
+void launch_setup(const SetupArgs& A, void*) {
+  std::function<void(EmuCtx&)> f = [&](EmuCtx& c) { body_setup(c, A); };
+  emu_launch((int)((A.n + SETUP_T - 1) / SETUP_T), SETUP_T, 0, f);
+}
+
 struct EmuEvent {
   std::chrono::steady_clock::time_point t;
 };
 void* dev_event_create() { return new EmuEvent(); }
 void dev_event_destroy(void* e) { delete (EmuEvent*)e; }
 void dev_event_record(void* e, void*) { ((EmuEvent*)e)->t = std::chrono::steady_clock::now(); }
+void dev_event_wait(void*) {}
 bool dev_event_done(void*) { return true; }  // emulated launches are synchronous
 bool dev_capture_begin(void*) { return false; }
 void* dev_capture_end(void*) { throw DeviceError(-3, "emulator: no graph capture"); }

@@ -43,7 +43,7 @@ namespace kw {
 // chirp w_n = exp(-i pi n^2 / N), X_k = w_k sum_n (x_n w_n) conj(w_(k-n)),
 // a circular convolution of length L >= 2N - 1 (L = 2^a 3^b 5^c) computed
 // with two length-L transforms in LDS; `chirp` (N entries) and `bspec`
-// (L entries: the length-L transform of the chirp filter conj(w_m),
+// (L entries: 1/L times the length-L transform of the chirp filter conj(w_m),
 // m = -(N-1) .. N-1, wrapped) are set, and the inverse uses their conjugates.
 struct FftPlan {
   int32_t N;   // length of the transform
@@ -582,8 +582,8 @@ KW_BODY void fft_stages_rt(Ctx& c, const FftPlan& pl, const TW& tw, int g, int G
 
 // Bluestein's transform of length N (see FftPlan) over the length-L stages:
 // the chirped input zero-padded to L, a forward transform, the product with
-// the filter's transform, an inverse transform, and the chirped outputs
-// scaled by 1/L; the inverse transform conjugates the chirp and the filter.
+// the filter's transform (which holds the 1/L), an inverse transform, and the
+// chirped outputs; the inverse transform conjugates the chirp and the filter.
 // Each thread reads and writes only its own elements n = g + i G between
 // barriers, as the plain runtime engine does.
 template <int NP, bool INV, class Ctx, class TW, class Src, class Dst>
@@ -621,12 +621,11 @@ KW_BODY void fft_bluestein(Ctx& c, const FftPlan& pl, const TW& tw, int g, int G
   }
   c.sync();
   fft_stages_rt<NP, true>(c, pl, tw, g, G, active, lds);
-  const float inv_l = 1.0f / (float)L;
 #pragma unroll
   for (int i = 0; i < kRtSlots; ++i) {
     const int n = g + i * G;
     if (active && n < N) {
-      const cf w = cscale(chirp(n), inv_l);
+      const cf w = chirp(n);
 #pragma unroll
       for (int j = 0; j < NP; ++j) dst(j, n, cmul(lds.get(j, n), w), i);
     }

@@ -183,6 +183,13 @@ void launch_ew(int nblocks, const Batch& B, const EwArgs& A, void* stream) {
   check(hipGetLastError(), "kernel launch");
 }
 
+void launch_k_setup(int nblocks, void* stream, const SetupArgs& A);
+void launch_setup(const SetupArgs& A, void* stream) {
+  if (A.n <= 0) return;
+  launch_k_setup((int)((A.n + SETUP_T - 1) / SETUP_T), stream, A);
+  check(hipGetLastError(), "kernel launch");
+}
+
 void* dev_event_create() {
   hipEvent_t e;
   check(hipEventCreate(&e), "hipEventCreate");
@@ -222,6 +229,7 @@ void dev_graph_destroy(void* x) {
   if (x) (void)hipGraphExecDestroy((hipGraphExec_t)x);
 }
 
+void dev_event_wait(void* e) { check(hipEventSynchronize((hipEvent_t)e), "hipEventSynchronize"); }
 bool dev_event_done(void* e) {
   const hipError_t r = hipEventQuery((hipEvent_t)e);
   if (r == hipErrorNotReady) return false;

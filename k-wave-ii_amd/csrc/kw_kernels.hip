@@ -1,7 +1,7 @@
 // gfx950 kernels.  This file is compiled once per (pass kind, fixed length)
 // variant (KW_KIND = 0..7 and KW_SIZE = 0 for runtime lengths or one of the
 // fixed lengths of kw_variants.h), or with KW_KIND = 8 for the elementwise
-// kernel, so that the variants build in parallel; each compile defines its
+// kernel and 9 for the set-up kernel, so that the variants build in parallel; each compile defines its
 // kernels and one host launcher.
 #include <hip/hip_runtime.h>
 
@@ -42,7 +42,17 @@ struct GpuCtx {
   const ProbDev* __restrict__ probs, const int32_t* __restrict__ tiles, int32_t nprob
 #define KW_KBATCH const Batch B{probs, tiles, nprob}
 
-#if KW_KIND == 8
+#if KW_KIND == 9
+
+__global__ __launch_bounds__(SETUP_T) void k_setup(SetupArgs A) {
+  GpuCtx c;
+  body_setup(c, A);
+}
+void launch_k_setup(int nb, void* s, const SetupArgs& A) {
+  hipLaunchKernelGGL(k_setup, dim3(nb), dim3(SETUP_T), 0, (hipStream_t)s, A);
+}
+
+#elif KW_KIND == 8
 
 __global__ __launch_bounds__(256) void k_ew(KW_KPARAMS, EwArgs A) {
   GpuCtx c;

@@ -16,18 +16,12 @@ namespace kw {
 // problem validation and set-up
 // ---------------------------------------------------------------------------
 
-static std::vector<float> to_float(const double* a, int64_t n) {
-  std::vector<float> v(n);
-  parallel_for(n, [&](int64_t i) { v[i] = (float)a[i]; });
-  return v;
-}
-
 static Field scalar_field(Sim& S, float v) {
   return Field{S.upload(std::vector<float>{v}), 0u};
 }
 
 static Field make_field(Sim& S, const double* a, double s, int64_t n) {
-  if (a) return Field{S.upload(to_float(a, n)), ~0u};
+  if (a) return Field{S.upload_map(a, n), ~0u};
   return scalar_field(S, (float)s);
 }
 
@@ -321,16 +315,16 @@ std::unique_ptr<Sim> create_sim(const kw_problem* pr_in, void* stream, Arena* ar
 
   // medium (rounded once from double)
   const int64_t n = G.ncell;
-  P.c0 = make_field(*S, pr->c0, pr->c0_scalar, n);
+  // (the sound speed with the absorption maps made of it, below)
+  const bool c0_maps = pr->c0 && !pr->alpha_coeff && pr->absorbing_flag != 0 && S->setup_on_device(n);
+  if (!c0_maps) P.c0 = make_field(*S, pr->c0, pr->c0_scalar, n);
   P.rho0 = make_field(*S, pr->rho0, pr->rho0_scalar, n);
   if (!pr->c0 && !(pr->c0_scalar > 0)) fail(KW_EINVAL, "sound speed must be positive");
   if (!pr->rho0 && !(pr->rho0_scalar > 0)) fail(KW_EINVAL, "density must be positive");
   for (int a = 0; a < dim; ++a) {
     const double* r = pr->rho0_sg[a] ? pr->rho0_sg[a] : pr->rho0;
     if (r) {
-      std::vector<float> inv(n);
-      parallel_for(n, [&](int64_t i) { inv[i] = (float)(1.0 / r[i]); });
-      P.rinv[a] = Field{S->upload(inv), ~0u};
+      P.rinv[a] = Field{S->upload_map(r, n, true), ~0u};
     } else {
       P.rinv[a] = scalar_field(*S, (float)(1.0 / pr->rho0_scalar));
     }
@@ -402,7 +396,23 @@ std::unique_ptr<Sim> create_sim(const kw_problem* pr_in, void* stream, Arena* ar
       const double an = a * conv;
       return s_eta * (2.0 * an * std::pow(c, y) * std::tan(kPi * y / 2));
     };
-    if (pr->alpha_coeff || pr->c0) {
+    if (c0_maps) {
+      const double an = pr->alpha_coeff_scalar * conv;
+      SetupArgs a{};
+      a.kind = SETUP_C0;
+      for (float*& o : a.out) o = S->alloc<float>((size_t)n);
+      a.tau = no_abs ? 0.0 : s_tau * (-2.0 * an);
+      a.tau_expo = P.eos == EOS_STOKES ? 1.0 : y - 1;
+      a.eta = no_disp || P.eos == EOS_STOKES ? 0.0 : s_eta * (2.0 * an * std::tan(kPi * y / 2));
+      a.eta_expo = y;
+      P.c0 = Field{a.out[0], ~0u};
+      P.tau = Field{a.out[1], ~0u};
+      if (P.eos == EOS_ABSORBING)
+        P.eta = Field{a.out[2], ~0u};
+      else
+        S->release(a.out[2]), a.out[2] = nullptr;
+      S->setup_map(pr->c0, n, a);
+    } else if (pr->alpha_coeff || pr->c0) {
       std::vector<float> tv(n), ev(n);
       parallel_for(n, [&](int64_t i) {
         const double a = pr->alpha_coeff ? pr->alpha_coeff[i] : pr->alpha_coeff_scalar;
@@ -509,14 +519,17 @@ std::unique_ptr<Sim> create_sim(const kw_problem* pr_in, void* stream, Arena* ar
     return std::sqrt(acc);
   };
   const double fit = rounding_of(*pr, dt);
-  P.kappa = S->spectral_table([&](int ix, int iy, int iz) {
+  const bool dev_tables = S->setup_on_device(G.nspec);
+  if (dev_tables) P.kappa = S->setup_table(SETUP_SINC, cref, dt, use_k, 0.0, Ntot / fit);
+  else P.kappa = S->spectral_table([&](int ix, int iy, int iz) {
     return (use_k ? sinc(cref * kmag(ix, iy, iz) * dt / 2) : 1.0) * fit / Ntot;
   });
   if (S->axisym) {
     // the radial divergence adds shift_y^- κ fft(u_y / r) (kspaceFirstOrderAS.m:
     // 954-969): κ times the y shift (which carries the 1/(Nx Ny) of the
     // round trip) in one last-axis pass
-    S->as_kappa = S->spectral_table([&](int ix, int iy, int iz) {
+    if (dev_tables) S->as_kappa = S->setup_table(SETUP_SINC, cref, dt, use_k, 0.0, 1.0 / fit);
+    else S->as_kappa = S->spectral_table([&](int ix, int iy, int iz) {
       return (use_k ? sinc(cref * kmag(ix, iy, iz) * dt / 2) : 1.0) * fit;
     });
     // ir: + on the copies that hold u_r, - on the mirrored ones, so that
@@ -569,12 +582,14 @@ std::unique_ptr<Sim> create_sim(const kw_problem* pr_in, void* stream, Arena* ar
       const int mz = dim == 3 ? (G.Nz - iz) % G.Nz : 0;
       return 0.5 * (at(ix, iy, iz) + at((G.Nx - ix) % G.Nx, (G.Ny - iy) % G.Ny, mz));
     };
-    P.nabla1 = S->spectral_table([&](int ix, int iy, int iz) {
+    if (dev_tables && !af && !no_abs) P.nabla1 = S->setup_table(SETUP_POW, cref, dt, true, y - 2, Ntot);
+    else P.nabla1 = S->spectral_table([&](int ix, int iy, int iz) {
       if (no_abs) return 0.0;
       const double v = std::pow(kmag(ix, iy, iz), y - 2);
       return std::isinf(v) ? 0.0 : v * filt(ix, iy, iz) / Ntot;
     });
-    P.nabla2 = S->spectral_table([&](int ix, int iy, int iz) {
+    if (dev_tables && !af && !no_disp) P.nabla2 = S->setup_table(SETUP_POW, cref, dt, true, y - 1, Ntot);
+    else P.nabla2 = S->spectral_table([&](int ix, int iy, int iz) {
       if (no_disp) return 0.0;
       const double v = std::pow(kmag(ix, iy, iz), y - 1);
       return std::isinf(v) ? 0.0 : v * filt(ix, iy, iz) / Ntot;
@@ -615,11 +630,13 @@ std::unique_ptr<Sim> create_sim(const kw_problem* pr_in, void* stream, Arena* ar
                            if (P.srcu[a].len > 0 && P.srcu[a].mode == SRC_ADDITIVE) return true;
                          return false;
                        }();
-  if (need_sk)
+  if (need_sk && dev_tables)
+    S->skappa = S->setup_table(SETUP_COS, cref, dt, use_k, 0.0, Ntot);
+  else if (need_sk)
     S->skappa = S->spectral_table([&](int ix, int iy, int iz) {
       return (use_k ? std::cos(cref * kmag(ix, iy, iz) * dt / 2) : 1.0) / Ntot;
     });
-  if (S->has_p0) S->p0 = S->upload(to_float(pr->p0, n));
+  if (S->has_p0) S->p0 = S->upload_map(pr->p0, n);
 
   // time reversal data and map
   if (S->time_rev) {
@@ -627,7 +644,7 @@ std::unique_ptr<Sim> create_sim(const kw_problem* pr_in, void* stream, Arena* ar
     for (int64_t i = 0; i < S->nsens; ++i)
       map[S->full_mask ? i : (int64_t)pr->sensor_mask_index[i] - 1] = (int32_t)i;
     P.tr_map = S->upload(map);
-    P.tr_data = S->upload(to_float(pr->time_reversal_boundary_data, S->nsens * pr->Nt));
+    P.tr_data = S->upload_map(pr->time_reversal_boundary_data, S->nsens * pr->Nt);
   }
   // sensor outputs
   if (S->nsens > 0 && !S->time_rev) {
@@ -801,6 +818,7 @@ std::unique_ptr<Sim> create_sim(const kw_problem* pr_in, void* stream, Arena* ar
   prep(pr->p_source, P.srcp, S->p_grid);
   for (int a = 0; a < dim; ++a) prep(pr->u_source[a], P.srcu[a], S->u_grid[a]);
   if (changed) dev_h2d(S->dP, &S->P, sizeof(ProbDev), S->stream);
+  S->end_staging();
   dev_sync(S->stream);
   return S;
 }
@@ -1557,7 +1575,8 @@ static void smooth(int dim, const int64_t N[3], const double* in, const double* 
     const int64_t wz = dim == 3 ? (iz + Nd[2] / 2) % Nd[2] : 0;
     return win[wx + (int64_t)Nd[0] * (wy + (int64_t)Nd[1] * wz)] / Ntot;
   });
-  float* f = S->upload(to_float(in, G.ncell));
+  float* f = S->upload_map(in, G.ncell);
+  S->end_staging();
   PassArgs a = bufs(1, 0);
   a.real[0] = f;
   S->pass(PK_X_R2C, a);

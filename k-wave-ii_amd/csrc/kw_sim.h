@@ -113,20 +113,21 @@ inline std::vector<double> pml_profile(int N, double d, double dt, double c, int
   return v;
 }
 
-// exp(-i a) in single precision: of the neighbours of the rounded cosine and
-// sine, the pair whose magnitude is nearest 1, a tenth of the angle's error
-// added.  A step's transforms come in pairs, forward and inverse, whose
-// angles cancel while magnitudes accumulate over the steps.
-inline cf root_of_unity(double a) {
-  const double c = std::cos(a), s = -std::sin(a);
+// A complex constant in single precision: of the neighbours of the rounded
+// parts, the pair whose magnitude is nearest, a tenth of the angle's error
+// added.  A step's transforms come in pairs, forward and inverse, whose angles
+// cancel while magnitudes accumulate over the steps.
+inline cf round_magnitude(std::complex<double> v) {
+  const double c = v.real(), s = v.imag(), r = std::abs(v);
   cf best{(float)c, (float)s};
-  if (best.x == 0.f || best.y == 0.f || std::fabs(c) < 1e-7 || std::fabs(s) < 1e-7) return best;
-  double least = 1e9;
+  if (std::fabs(c) < 1e-7 * r || std::fabs(s) < 1e-7 * r) return best;
+  double least = 1e300;
   for (int i = -1; i <= 1; ++i)
     for (int j = -1; j <= 1; ++j) {
-      const float x = i == 0 ? (float)c : std::nextafter((float)c, i * 2.f);
-      const float y = j == 0 ? (float)s : std::nextafter((float)s, j * 2.f);
-      const double m = ((double)x * x + (double)y * y - 1.0) / 2, t = (double)y * c - (double)x * s;
+      const float x = i == 0 ? (float)c : std::nextafter((float)c, i * 1e30f);
+      const float y = j == 0 ? (float)s : std::nextafter((float)s, j * 1e30f);
+      const double m = std::hypot((double)x, (double)y) - r;
+      const double t = ((double)y * c - (double)x * s) / r;
       const double e = std::fabs(m) + 0.1 * std::fabs(t);
       if (e < least) {
         least = e;
@@ -315,6 +316,14 @@ struct Sim {
   std::vector<void*> ev_free;
 
   ~Sim() {
+    if (staging) {
+      // creation failed: the kernels may still read the chunks
+      try {
+        dev_sync(stream);
+      } catch (...) {
+      }
+      staging.reset();
+    }
     for (auto& e : ev_used) {
       dev_event_destroy(e.first);
       dev_event_destroy(e.second);
@@ -366,6 +375,111 @@ struct Sim {
     T* d = alloc<T>(v.size());
     dev_h2d(d, v.data(), v.size() * sizeof(T), stream);
     return d;
+  }
+
+  // Set-up on the device (kw_setup.h) from this many elements; below it the
+  // host's loops and copies are shorter than a chunk buffer's allocation.
+  // Not in an arena, whose callers allocate nothing.
+  static constexpr int64_t kSetupMin = 1 << 16;
+  bool setup_on_device(int64_t n) const { return !arena && n >= kSetupMin; }
+
+  // Two pinned host chunks, alive while a simulation is created: one fills
+  // while the map kernel reads the other over the bus.
+  struct Staging {
+    size_t chunk;  // doubles
+    double* pin[2] = {nullptr, nullptr};
+    void* ev[2] = {nullptr, nullptr};
+    bool used[2] = {false, false};
+    int next = 0;
+    explicit Staging(size_t n) : chunk(std::min(n, (size_t)1 << 20)) {
+      try {
+        for (int i = 0; i < 2; ++i) {
+          pin[i] = (double*)dev_host_alloc(chunk * sizeof(double));
+          ev[i] = dev_event_create();
+        }
+      } catch (...) {
+        free_all();
+        throw;
+      }
+    }
+    ~Staging() { free_all(); }
+    Staging(const Staging&) = delete;
+    Staging& operator=(const Staging&) = delete;
+    void free_all() {
+      for (int i = 0; i < 2; ++i) {
+        if (pin[i]) dev_host_free(pin[i]);
+        if (ev[i]) dev_event_destroy(ev[i]);
+      }
+    }
+  };
+  std::unique_ptr<Staging> staging;
+  void end_staging() {
+    if (!staging) return;
+    dev_sync(stream);  // the kernels have read the chunks
+    staging.reset();
+  }
+
+  // the map kernel `a` over n doubles in host memory, chunk by chunk
+  void setup_map(const double* src, int64_t n, SetupArgs a) {
+    if (!staging) staging.reset(new Staging((size_t)n));
+    Staging& s = *staging;
+    for (int64_t at = 0; at < n; at += (int64_t)s.chunk) {
+      const int64_t m = std::min<int64_t>((int64_t)s.chunk, n - at);
+      const int i = s.next;
+      s.next ^= 1;
+      if (s.used[i]) dev_event_wait(s.ev[i]);
+      const int64_t slice = 1 << 15;
+      double* to = s.pin[i];
+      parallel_for((m + slice - 1) / slice, [=](int64_t k) {
+        const int64_t lo = k * slice, len = std::min(slice, m - lo);
+        std::memcpy(to + lo, src + at + lo, (size_t)len * sizeof(double));
+      }, slice);
+      SetupArgs c = a;
+      c.n = m;
+      c.src = to;
+      for (int o = 0; o < 3; ++o)
+        if (c.out[o]) c.out[o] = a.out[o] + at;
+      launch_setup(c, stream);
+      dev_event_record(s.ev[i], stream);
+      s.used[i] = true;
+    }
+  }
+  // n doubles as a single-precision device array (or their reciprocals)
+  float* upload_map(const double* src, int64_t n, bool inverse = false) {
+    if (!setup_on_device(n)) {
+      std::vector<float> v((size_t)n);
+      parallel_for(n, [&](int64_t i) { v[i] = (float)(inverse ? 1.0 / src[i] : src[i]); });
+      return upload(v);
+    }
+    SetupArgs a{};
+    a.kind = inverse ? SETUP_INV : SETUP_F32;
+    a.out[0] = alloc<float>((size_t)n);
+    setup_map(src, n, a);
+    return a.out[0];
+  }
+
+  // Table of the set-up kernel's kind (SETUP_SINC, SETUP_COS, SETUP_POW)
+  // divided by ntot, in the order of spectral_table
+  float* setup_table(int kind, double c_ref, double dt, bool use_k, double expo, double ntot) {
+    SetupArgs a{};
+    a.kind = kind;
+    a.dim = G.dim;
+    a.Nx = G.Nx;
+    a.Ny = G.Ny;
+    a.Nz = G.Nz;
+    a.Wm = G.Wm;
+    a.nyq = G.nyq;
+    a.Pn = P.Pl;
+    for (int k = 0; k < 3; ++k) a.d[k] = op.d[k];
+    a.c_ref = c_ref;
+    a.dt = dt;
+    a.use_k = use_k ? 1 : 0;
+    a.expo = expo;
+    a.ntot = ntot;
+    a.n = (int64_t)ll.nb * (G.dim == 3 ? G.Nz : G.Ny) * P.Pl;
+    a.out[0] = alloc<float>((size_t)a.n);
+    launch_setup(a, stream);
+    return a.out[0];
   }
 
   Batch batch() const { return Batch{dP, d_tile0, 1}; }
@@ -596,7 +710,11 @@ struct Sim {
     for (size_t i = 0; i < r.size(); ++i) pl.radix[i] = r[i];
     std::vector<cf> tw(L);
     for (int j = 0; j < L; ++j) {
-      tw[j] = root_of_unity(2.0 * kPi * (double)j / (double)L);
+      const double a = 2.0 * kPi * (double)j / (double)L;
+      const std::complex<double> w(std::cos(a), -std::sin(a));
+      // (the chirp-z transform's own pair has a product between them, so
+      // there the angles count: rounded to nearest)
+      tw[j] = direct ? round_magnitude(w) : cf{(float)w.real(), (float)w.imag()};
     }
     pl.tw = upload(tw);
     if (!direct) {
@@ -619,8 +737,8 @@ struct Sim {
         B[k] = acc;
       }, N);
       std::vector<cf> ch(N), bs(L);
-      for (int n = 0; n < N; ++n) ch[n] = cf{(float)w[n].real(), (float)w[n].imag()};
-      for (int k = 0; k < L; ++k) bs[k] = cf{(float)B[k].real(), (float)B[k].imag()};
+      for (int n = 0; n < N; ++n) ch[n] = round_magnitude(w[n]);
+      for (int k = 0; k < L; ++k) bs[k] = round_magnitude(B[k] / (double)L);
       pl.chirp = upload(ch);
       pl.bspec = upload(bs);
     }

@@ -1,0 +1,53 @@
+"""Operators and medium maps built on the device (grids of 2^16 cells and
+more) against the host's: kw_run builds them on the device, kw_run_noalloc,
+which may not allocate a chunk, on the host.  Both evaluate in double
+precision and round once, so an entry differs at most in its last single
+bit, and a few steps at most to 1e-6 of the largest value."""
+
+import numpy as np
+import pytest
+
+import cases
+
+KINDS = ["power", "no_dispersion", "no_absorption", "stokes", "alpha_map", "lossless_ragged"]
+
+
+def _case(kind, shape):
+    rng = np.random.default_rng(len(kind))
+    med = {"sound_speed": 1500 + 50 * rng.random(shape), "density": 1000 + 50 * rng.random(shape)}
+    if kind != "lossless_ragged":
+        med.update(alpha_coeff=0.75, alpha_power=1.5, BonA=6 + rng.random(shape))
+    if kind in ("no_dispersion", "no_absorption", "stokes"):
+        med["alpha_mode"] = kind
+    if kind == "alpha_map":
+        med["alpha_coeff"] = 0.5 + rng.random(shape)
+    src = np.zeros(shape)
+    src[tuple(n // 2 for n in shape)] = 1
+    return {"dim": len(shape), "shape": shape, "dx": 1e-4, "Nt": 5, "dt": 1.5e-8, "medium": med,
+            "source": {"p_mask": src, "p": np.array([[1.0, -2.0, 1.5, 0.5, -1.0]]), "p_mode": "additive"},
+            "sensor": {"mask": np.ones(shape), "record": ["p_final", "p_max", "u_final"]},
+            "opts": {"PMLSize": 6, "Smooth": False}}
+
+
+def _check(lib, kind):
+    shape = (49, 37, 41) if kind == "lossless_ragged" else (256, 300)
+    pp = cases.prepared(_case(kind, shape))
+    dev = cases.run_entry(lib, "kw_run", pp)
+    host = cases.run_entry(lib, "kw_run_noalloc", pp)
+    for k in host:
+        g, w = np.asarray(dev[k], dtype=np.float64), np.asarray(host[k], dtype=np.float64)
+        assert np.max(np.abs(w)) > 0 and np.max(np.abs(g - w)) <= 1e-6 * np.max(np.abs(w)), (kind, k)
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_device_setup_emu(kind):
+    from kwhip import _abi
+    with _abi._backend_override("emu"):
+        _check(_abi.load("emu"), kind)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", KINDS)
+def test_device_setup_hip(kind, hip_lib):
+    _check(hip_lib, kind)
+
