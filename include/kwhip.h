@@ -457,6 +457,15 @@ int kw_run_file(const char* input_file, const char* output_file, uint32_t record
 int kw_smooth(int32_t dim, const int64_t N[3], const double* in, const double* win,
               double* out, char* err, size_t errlen);
 
+/* Host helper: a row-major grid (last axis fastest) as the column-major array
+ * that a kw_problem takes, on up to 16 host threads.  With `sg` not NULL,
+ * sg[a] (a < dim) receives the values half a cell further along axis a,
+ * v + 0.5 (v_next - v), the last plane unchanged
+ * (kspaceFirstOrder3D.m:585-607).  `out` may be `in` when that is column-major
+ * already. */
+int kw_layout(int32_t dim, const int64_t N[3], const double* in, double* out,
+              double* const sg[3], char* err, size_t errlen);
+
 #ifdef __cplusplus
 }
 #endif

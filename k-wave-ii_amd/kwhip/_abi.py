@@ -213,6 +213,8 @@ def load(backend: str = "hip") -> C.CDLL:
     lib.kw_sim_destroy.argtypes = [C.c_void_p]
     lib.kw_sim_step_timed.argtypes = [C.c_void_p, C.c_int64, P(C.c_double), P(KernelStats)] + err
     lib.kw_smooth.argtypes = [C.c_int32, P(C.c_int64), c_double_p, c_double_p, c_double_p] + err
+    lib.kw_layout.argtypes = [C.c_int32, P(C.c_int64), c_double_p, c_double_p,
+                              P(c_double_p)] + err
     lib.kw_save_problem.argtypes = [P(Problem), C.c_char_p] + err
     lib.kw_run_file.argtypes = [C.c_char_p, C.c_char_p, C.c_uint32, C.c_int64] + err
     lib.kw_engine_create.argtypes = [P(EngineConfig), P(C.c_void_p)] + err
@@ -258,41 +260,43 @@ def as_f64(a):
     return None if a is None else np.ascontiguousarray(a, dtype=np.float64)
 
 
-_FLAT_POOL = None
-
-
-def host_pool():
-    """A few host threads for slab-parallel NumPy work on large grids (NumPy
-    releases the GIL inside its copy and arithmetic loops)."""
-    global _FLAT_POOL
-    if _FLAT_POOL is None:
-        from concurrent.futures import ThreadPoolExecutor
-        _FLAT_POOL = ThreadPoolExecutor(max_workers=8)
-    return _FLAT_POOL
-
-
-def by_slabs(fn, n, k=8):
-    """fn(lo, hi) over k slabs of range(n), on the host pool."""
-    k = max(1, min(k, n))
-    bounds = [n * i // k for i in range(k + 1)]
-    list(host_pool().map(lambda i: fn(bounds[i], bounds[i + 1]), range(k)))
+def _layout(a, out, sg):
+    sgp = None if sg is None else (c_double_p * 3)(*[dptr(s) for s in sg])
+    call(load(active_backend()).kw_layout, C.c_int32(a.ndim),
+         (C.c_int64 * 3)(*a.shape, *([1] * (3 - a.ndim))), dptr(a), dptr(out), sgp)
 
 
 def fortran_flat(a):
-    """Column-major (MATLAB) flattening of a grid array as float64.  Large
-    row-major grids are transposed by slabs of the last axis on a few host
-    threads (NumPy releases the GIL while it copies), several times faster
-    than one strided copy."""
+    """Column-major (MATLAB) flattening of a grid array as float64; large
+    row-major grids go through the library's threaded transpose."""
     a = np.asarray(a, dtype=np.float64)
-    if a.ndim < 2 or a.size < (1 << 20) or a.flags.f_contiguous:
+    if a.ndim < 2 or a.size < (1 << 16) or not a.flags.c_contiguous:
         return np.ascontiguousarray(a.ravel(order="F"))
-    out = np.empty(a.shape, dtype=np.float64, order="F")
+    out = np.empty(a.size)
+    _layout(a, out, None)
+    return out
 
-    def part(lo, hi):
-        out[..., lo:hi] = a[..., lo:hi]
 
-    by_slabs(part, a.shape[-1])
-    return out.ravel(order="F")  # a view: out is column-major
+def fortran_staggered(a):
+    """fortran_flat(a) and, per axis, the values half a cell further along it
+    (v + 0.5 (v_next - v), the last plane unchanged), flattened alike."""
+    a = np.asarray(a, dtype=np.float64)
+    if a.size >= (1 << 16):
+        sg = [np.empty(a.size) for _ in range(a.ndim)]
+        if a.flags.c_contiguous:
+            flat = np.empty(a.size)
+            _layout(a, flat, sg)
+        else:
+            flat = fortran_flat(a)
+            _layout(flat.reshape(a.shape, order="F"), flat, sg)
+        return flat, sg
+    sg = []
+    for ax in range(a.ndim):
+        s = a.copy()
+        lo, hi = ((slice(None),) * ax + (slice(*r),) for r in ((0, -1), (1, None)))
+        s[lo] = a[lo] + 0.5 * (a[hi] - a[lo])
+        sg.append(fortran_flat(s))
+    return fortran_flat(a), sg
 
 
 def backend_name(lib) -> str:

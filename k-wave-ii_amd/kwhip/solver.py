@@ -368,6 +368,9 @@ def check_stability(kgrid: kWaveGrid, c, c_ref, medium):
     y = 2.0 if mode == "stokes" else float(np.asarray(_get(medium, "alpha_power")))
     a_np = 100.0 * np.asarray(alpha, dtype=np.float64) * (1e-6 / (2 * math.pi)) ** y / \
         (20.0 * math.log10(math.e))
+    if a_np.size == 1:
+        # tau and eta are powers of c alone, so their extremes are at c's
+        c = np.array([float(np.min(c)), c_max])
     tau = 0.0 if mode == "no_absorption" else -2.0 * a_np * c ** (y - 1)
     eta = 0.0 if mode == "no_dispersion" else 2.0 * a_np * c ** y * math.tan(math.pi * y / 2)
     tau_min, eta_min = float(np.min(tau)), float(np.min(eta))
@@ -400,7 +403,8 @@ def _find(mask) -> np.ndarray:
     sorted, which avoids a transposed copy of the whole grid."""
     m = np.asarray(mask)
     if m.ndim > 1 and np.count_nonzero(m) * 8 < m.size:
-        lin = np.ravel_multi_index(np.nonzero(m), m.shape, order="F")
+        at = np.unravel_index(np.flatnonzero(m.ravel() != 0), m.shape)
+        lin = np.ravel_multi_index(at, m.shape, order="F")
         lin.sort()
         return lin
     return np.flatnonzero(np.asarray(m != 0).ravel(order="F"))
@@ -810,35 +814,9 @@ def prepare(kgrid: kWaveGrid, medium, source, sensor, dim: int, opts: dict) -> P
     # -- staggered density (kspaceFirstOrder3D.m:585-607) ----------------------
     use_sg = bool(opts.get("UseSG", True))
     rho_sg = [None] * 3
+    rho_flat = None
     if rho.size > 1 and use_sg:
-        # computed on the column-major copy, so every array is contiguous and
-        # its flattening free
-        rho_f = _abi.fortran_flat(rho).reshape(shape, order="F")
-        last = dim - 1
-        for ax in range(dim):
-            sg = np.empty(shape, dtype=np.float64, order="F")
-
-            def part(z0, z1, ax=ax, sg=sg):
-                # slab z0:z1 of the last axis; along the last axis the
-                # neighbour plane may lie in the next slab (read only)
-                a = rho_f[..., z0:z1]
-                o = sg[..., z0:z1]
-                o[...] = a
-                if ax == last:
-                    z1i = min(z1, shape[last] - 1)
-                    if z1i > z0:
-                        lo = rho_f[..., z0:z1i]
-                        o[..., :z1i - z0] = lo + 0.5 * (rho_f[..., z0 + 1:z1i + 1] - lo)
-                else:
-                    sl_lo = [slice(None)] * dim
-                    sl_hi = [slice(None)] * dim
-                    sl_lo[ax] = slice(0, -1)
-                    sl_hi[ax] = slice(1, None)
-                    sl_lo, sl_hi = tuple(sl_lo), tuple(sl_hi)
-                    o[sl_lo] = a[sl_lo] + 0.5 * (a[sl_hi] - a[sl_lo])
-
-            _abi.by_slabs(part, shape[last])
-            rho_sg[ax] = sg.ravel(order="F")
+        rho_flat, rho_sg[:dim] = _abi.fortran_staggered(rho)
 
     # -- fill the kw_problem ---------------------------------------------------
     pr.dim = dim
@@ -855,7 +833,7 @@ def prepare(kgrid: kWaveGrid, medium, source, sensor, dim: int, opts: dict) -> P
 
     a, s_ = grid_or_scalar(c)
     pr.c0, pr.c0_scalar = _abi.dptr(a), s_
-    a, s_ = grid_or_scalar(rho)
+    a, s_ = grid_or_scalar(rho) if rho_flat is None else (pp.hold(rho_flat), 0.0)
     pr.rho0, pr.rho0_scalar = _abi.dptr(a), s_
     for ax in range(3):
         pr.rho0_sg[ax] = _abi.dptr(pp.hold(rho_sg[ax]))
@@ -951,7 +929,7 @@ def prepare(kgrid: kWaveGrid, medium, source, sensor, dim: int, opts: dict) -> P
         pr.record_flags = rec_flags
         pr.record_start_index = record_start
         if info.time_rev:
-            pr.time_reversal_boundary_data = _abi.dptr(pp.hold(np.ascontiguousarray(tr_data.ravel(order="F"))))
+            pr.time_reversal_boundary_data = _abi.dptr(pp.hold(_abi.fortran_flat(tr_data)))
     info.n_sensor = n_sens if info.use_sensor else 0
     info.n_rec = (Nt - record_start + 1) if (info.use_sensor and not info.time_rev) else 0
     info.data_recast = bool(opts.get("DataRecast", False))

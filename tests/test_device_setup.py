@@ -2,7 +2,8 @@
 more) against the host's: kw_run builds them on the device, kw_run_noalloc,
 which may not allocate a chunk, on the host.  Both evaluate in double
 precision and round once, so an entry differs at most in its last single
-bit, and a few steps at most to 1e-6 of the largest value."""
+bit, and a few steps at most to 1e-6 of the largest value.  The staggered
+column-major layout of a density map is checked against NumPy bit for bit."""
 
 import numpy as np
 import pytest
@@ -51,3 +52,18 @@ def test_device_setup_emu(kind):
 def test_device_setup_hip(kind, hip_lib):
     _check(hip_lib, kind)
 
+
+@pytest.mark.parametrize("order", ["C", "F"])
+@pytest.mark.parametrize("shape", [(70001,), (300, 257), (67, 33, 41), (5, 4, 3)])
+def test_layout(shape, order):
+    from kwhip import _abi
+    a = np.asarray(np.random.default_rng(1).random(shape), order=order)
+    with _abi._backend_override("emu"):
+        flat, sg = _abi.fortran_staggered(a)
+        assert np.array_equal(_abi.fortran_flat(a), a.ravel(order="F"))
+    assert np.array_equal(flat, a.ravel(order="F"))
+    for ax in range(a.ndim):
+        m = np.moveaxis(a, ax, 0)
+        want = m.copy()
+        want[:-1] = m[:-1] + 0.5 * (m[1:] - m[:-1])
+        assert np.array_equal(sg[ax], np.moveaxis(want, 0, ax).ravel(order="F"))
