@@ -316,13 +316,13 @@ void emu_lds_access(const cf* p, bool write, const cf* value) {
   if (!ordered) lds_fault("read without a barrier after the write of lane", R->bid, me, i, w);
 }
 
-template <class Sel, class SelX>
+template <class Sel, class SelX, class SelY>
 static void emu_pass(PassKind kind, int dim, int nblocks, int threads, size_t lds_bytes,
                      const Batch& B, const PassArgs& A) {
   std::function<void(EmuCtx&)> f;
   switch (kind) {
-    case PK_YFWD: f = [&](EmuCtx& c) { body_ypass<false, Sel>(c, B, A); }; break;
-    case PK_YINV: f = [&](EmuCtx& c) { body_ypass<true, Sel>(c, B, A); }; break;
+    case PK_YFWD: f = [&](EmuCtx& c) { body_ypass<false, SelY>(c, B, A); }; break;
+    case PK_YINV: f = [&](EmuCtx& c) { body_ypass<true, SelY>(c, B, A); }; break;
     case PK_SPEC:
       if (spec_is_aux(A))
         f = [&](EmuCtx& c) { body_spec<Sel, true>(c, B, A); };
@@ -351,9 +351,9 @@ static void emu_pass(PassKind kind, int dim, int nblocks, int threads, size_t ld
 void launch_pass(PassKind kind, int fixed, int dim, int nblocks, int threads, size_t lds_bytes,
                  const Batch& B, const PassArgs& A, void*) {
   switch (fixed) {
-    case 0: emu_pass<PlanRt, PlanRt>(kind, dim, nblocks, threads, lds_bytes, B, A); break;
+    case 0: emu_pass<PlanRt, PlanRt, PlanRt>(kind, dim, nblocks, threads, lds_bytes, B, A); break;
 #define KW_EMU_SIZE(SIZE) \
-    case SIZE: emu_pass<PlanCt<SIZE>, PlanCtX<SIZE>>(kind, dim, nblocks, threads, lds_bytes, B, A); break;
+    case SIZE: emu_pass<PlanCt<SIZE>, PlanCtX<SIZE>, PlanCtY<SIZE>>(kind, dim, nblocks, threads, lds_bytes, B, A); break;
     KW_EMU_FIXED_SIZES(KW_EMU_SIZE)
 #undef KW_EMU_SIZE
     default: throw DeviceError(-3, "no kernel variant for this length");

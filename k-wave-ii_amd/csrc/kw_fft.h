@@ -94,18 +94,19 @@ KW_HOSTDEV constexpr void ct_search(int N, int rest, int G, int emax, CtPlan cur
 
 // strided plan of length N with G threads, at most 12 elements per thread,
 // largest radix first (the first stage has no twiddles)
-KW_HOSTDEV constexpr CtPlan ct_strided(int N, int G) {
+KW_HOSTDEV constexpr CtPlan ct_strided(int N, int G, int most = 12) {
   CtPlan best;
-  ct_search(N, N, G, 12, CtPlan{}, 0, 12, best);
+  ct_search(N, N, G, most, CtPlan{}, 0, 12, best);
   return best;
 }
 // threads per pencil of the strided plan: the least work over all lanes,
 // then the most threads (half the elements per thread and five stages instead
 // of four took the last axis of 1024 x 1024 from 21 to 23 us)
-KW_HOSTDEV constexpr int strided_threads(int N) {
+KW_HOSTDEV constexpr int strided_threads(int N, int most = 12) {
   int g = 0, work = 1 << 30;
-  for (int G = (N + 11) / 12; G <= (N + 7) / 8; ++G) {
-    const CtPlan p = ct_strided(N, G);
+  for (int G = (N + most - 1) / most; G <= (N + 5) / 6; ++G) {
+    if (G > (N + 7) / 8 && g > 0) break;
+    const CtPlan p = ct_strided(N, G, most);
     if (p.nst > 0 && p.cost * G <= work) {
       g = G;
       work = p.cost * G;
@@ -113,6 +114,12 @@ KW_HOSTDEV constexpr int strided_threads(int N) {
   }
   return g;
 }
+// The y passes of an axis above 256: at most eight elements per thread.  Their
+// blocks have 768 threads and more, of which a CU holds two only while a
+// thread's registers are few (384 = 12 8 4 on 48 threads: 224 us a forward
+// launch of 384^3, 167 as 8 8 6 on 64).
+KW_HOSTDEV constexpr int y_most(int N) { return N > 256 && strided_threads(N, 8) > 0 ? 8 : 12; }
+KW_HOSTDEV constexpr int y_threads(int N) { return strided_threads(N, y_most(N)); }
 // x plan: the stage that leaves a thread the fewest elements last, the
 // largest of the others first
 KW_HOSTDEV constexpr CtPlan ct_xplan(int N, int G) {
@@ -680,11 +687,11 @@ KW_BODY void last_slots_rt(const FftPlan& pl, int g, int G, bool, F& f) {
 // ---- fixed-length engine ------------------------------------------------------
 
 // N, threads per pencil G and the plan family (X: x passes) as constants
-template <int N_, int G_, bool X>
+template <int N_, int G_, bool X, int MOST = 12>
 struct CtShape {
   static constexpr int N = N_;
   static constexpr int G = G_;
-  static constexpr CtPlan plan = X ? ct_xplan(N, G) : ct_strided(N, G);
+  static constexpr CtPlan plan = X ? ct_xplan(N, G) : ct_strided(N, G, MOST);
   static constexpr int nst = plan.nst;
   static_assert(nst > 0, "length must factor into 2, 3 and 5");
   static constexpr int radix(int s) { return plan.r[s]; }
@@ -767,23 +774,6 @@ KW_BODY void last_slots_ct(int g, bool, F& f) {
 // A kernel body templated on a selector runs the runtime engine (PlanRt) or
 // the fixed-length engine (PlanCt<N>) for one axis.
 
-// What a source's first loads bring into registers and how an input is made
-// of it: sources that combine several loads name a Raw type and give raw(n)
-// and join(raw, n), so that the loads can be in flight before the combination
-// waits for them; any other source is called.
-template <class Src, class = void>
-struct SrcRaw {
-  using type = cf;
-  KW_BODY static cf raw(Src& s, int n) { return s(0, n); }
-  KW_BODY static cf join(Src&, const cf& r, int) { return r; }
-};
-template <class Src>
-struct SrcRaw<Src, std::void_t<typename Src::Raw>> {
-  using type = typename Src::Raw;
-  KW_BODY static type raw(Src& s, int n) { return s.raw(n); }
-  KW_BODY static cf join(Src& s, const type& r, int n) { return s.join(r, n); }
-};
-
 // Start of a block: `load_first` issues the loads of a transform's first
 // stage before the block has its twiddles, which that stage does not use, so
 // the two memory latencies overlap; `fft_pre` runs the transform from them.
@@ -854,20 +844,18 @@ struct PlanFixed {
   static constexpr bool twiddles_first = false;
   template <class Src>
   struct Pre {
-    typename SrcRaw<Src>::type v[Sh::first_slots];
+    cf v[Sh::first_slots];
   };
   template <class Src>
   KW_BODY static void load_first(int g, Src& src, Pre<Src>& pre) {
-    auto f = [&](int slot, int n) { pre.v[slot] = SrcRaw<Src>::raw(src, n); };
+    auto f = [&](int slot, int n) { pre.v[slot] = src(0, n); };
     first_slots_ct<Sh>(g, f);
   }
   template <int NP, bool INV, class Ctx, class TW, class Src, class Dst>
   KW_BODY static void fft_pre(Ctx& c, const FftPlan&, const TW& tw, int g, int, bool active,
-                              Src& src, Pre<Src>& pre, Dst& dst, const LdsPencils& lds) {
+                              Src&, Pre<Src>& pre, Dst& dst, const LdsPencils& lds) {
     static_assert(NP == 1, "one pencil");
-    auto held = [&](int, int n, int slot) -> cf {
-      return SrcRaw<Src>::join(src, pre.v[slot], n);
-    };
+    auto held = [&](int, int, int slot) -> cf { return pre.v[slot]; };
     fft_ct<Sh, 1, INV>(c, tw, g, active, held, dst, lds);
   }
   template <int NP, bool INV, class Ctx, class TW, class Src, class Dst>
@@ -881,9 +869,11 @@ struct PlanFixed {
   }
 };
 
-// the plan of the strided and last-axis passes for a fixed length
+// the plans of the last-axis and the strided y passes for a fixed length
 template <int N>
 using PlanCt = PlanFixed<CtShape<N, strided_threads(N), false>>;
+template <int N>
+using PlanCtY = PlanFixed<CtShape<N, y_threads(N), false, y_most(N)>>;
 
 // the plan of the x passes for a fixed length
 template <int N>

@@ -74,7 +74,11 @@ void launch_k_ew(int nb, int T, size_t lds, void* s, const Batch& B, const EwArg
 using Sel = PlanRt;
 using SelX = PlanRt;
 #else
+#if KW_KIND <= 1
+using Sel = PlanCtY<KW_SIZE>;
+#else
 using Sel = PlanCt<KW_SIZE>;
+#endif
 using SelX = PlanCtX<KW_SIZE>;
 #endif
 

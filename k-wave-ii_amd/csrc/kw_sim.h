@@ -658,7 +658,7 @@ struct Sim {
     // pencil, which a group of uneven sizes uses: see Group::rebuild)
     // strided y pass (3D): <= 1024 threads, LDS Ny twiddles + P*(Ny+1)
     if (G.dim == 3) {
-      const int Gy = fixed_len(PK_YFWD) ? strided_threads(G.Ny) : Gof(G.Ny);
+      const int Gy = fixed_len(PK_YFWD) ? y_threads(G.Ny) : Gof(G.Ny);
       const int Ly = stage_length(G.Ny);
       int P = std::max(1, std::min(pencils_env("KW_PENCILS_Y", tiles.y ? tiles.y : 16),
                                    1024 / std::max(Gy, Gof(G.Ny))));
