@@ -466,6 +466,12 @@ int kw_smooth(int32_t dim, const int64_t N[3], const double* in, const double* w
 int kw_layout(int32_t dim, const int64_t N[3], const double* in, double* out,
               double* const sg[3], char* err, size_t errlen);
 
+/* kw_layout for a grid in any order: element (x, y, z) at
+ * in[x stride[0] + y stride[1] + z stride[2]], strides in elements, of
+ * either sign or 0. */
+int kw_layout_strided(int32_t dim, const int64_t N[3], const int64_t stride[3], const double* in,
+                      double* out, double* const sg[3], char* err, size_t errlen);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1592,22 +1592,39 @@ static void smooth(int dim, const int64_t N[3], const double* in, const double* 
   for (int64_t i = 0; i < G.ncell; ++i) out[i] = h[i];
 }
 
-// kw_layout.  The transpose goes by tiles of kT x kT of the first and last
-// axis, so that reads and writes both run along whole cache lines: 256^3
-// doubles in 6.8 ms, 13.2 ms with the three staggered copies, where NumPy's
-// strided copies on eight threads took 16.5 ms for the transpose alone.
-static void layout(int dim, const int64_t N[3], const double* in, double* out,
-                   double* const sg[3]) {
-  constexpr int64_t kT = 32;
+// kw_layout and kw_layout_strided.  The transpose goes by tiles of kT x kT of
+// the first axis and the one that the input has closest together (whole rows
+// where that is the first axis itself), so that reads and writes both run
+// along whole cache lines.  256^3 doubles take 6.1 ms from row-major order, 5.6
+// cut out of a wider array and 7.1 with two axes exchanged; NumPy's strided copy
+// takes 25 and 78 for the last two, and by slabs on eight threads 18, 5.9 and
+// 15.  A thread gets at least kLayoutGrain elements: sixteen threads for the
+// 90,000 of 300 x 300 took 4.0 ms, one takes 0.04.
+constexpr int64_t kLayoutGrain = 1 << 17;
+
+static void layout(int dim, const int64_t N[3], const int64_t stride[3], const double* in,
+                   double* out, double* const sg[3]) {
   const int64_t nx = N[0], ny = dim == 3 ? N[1] : 1, nz = dim == 1 ? 1 : N[dim - 1];
-  const int64_t tx = (nx + kT - 1) / kT, tz = (nz + kT - 1) / kT;
-  // in[(x ny + y) nz + z] -> out[x + nx (y + ny z)]
-  if (in != out) parallel_for(ny * tx * tz, [=](int64_t i) {
-    const int64_t z0 = i % tz * kT, y = i / tz % ny, x0 = i / (tz * ny) * kT;
-    const int64_t x1 = std::min(nx, x0 + kT), z1 = std::min(nz, z0 + kT);
-    for (int64_t z = z0; z < z1; ++z)
-      for (int64_t x = x0; x < x1; ++x) out[x + nx * (y + ny * z)] = in[(x * ny + y) * nz + z];
-  }, kT * kT);
+  const int64_t sx = stride[0], sy = dim == 3 ? stride[1] : 0, sz = dim == 1 ? 0 : stride[dim - 1];
+  // in[x sx + y sy + z sz] -> out[x + nx (y + ny z)], y or z as the tiles'
+  // second axis b and the other as c (rows go in the order of the output)
+  const bool rows_in = (ny == 1 || std::abs(sx) <= std::abs(sy)) &&
+                       (nz == 1 || std::abs(sx) <= std::abs(sz));
+  const bool by_y = rows_in || (ny > 1 && (nz == 1 || std::abs(sy) < std::abs(sz)));
+  const int64_t nb = by_y ? ny : nz, nc = by_y ? nz : ny;
+  const int64_t sb = by_y ? sy : sz, sc = by_y ? sz : sy;
+  const int64_t ob = by_y ? nx : nx * ny, oc = by_y ? nx * ny : nx;
+  const int64_t tx = rows_in ? nx : 32, tb = rows_in ? 1 : 32;
+  const int64_t mx = (nx + tx - 1) / tx, mb = (nb + tb - 1) / tb;
+  if (in != out) parallel_for(nc * mx * mb, [=](int64_t i) {
+    const int64_t b0 = i % mb * tb, c = i / mb % nc, x0 = i / (mb * nc) * tx;
+    const int64_t x1 = std::min(nx, x0 + tx), b1 = std::min(nb, b0 + tb);
+    for (int64_t b = b0; b < b1; ++b) {
+      const double* v = in + b * sb + c * sc;
+      double* o = out + b * ob + c * oc;
+      for (int64_t x = x0; x < x1; ++x) o[x] = v[x * sx];
+    }
+  }, tx * tb, kLayoutGrain);
   if (!sg) return;
   const int64_t rows = ny * nz;
   parallel_for(rows, [=](int64_t r) {
@@ -1626,7 +1643,7 @@ static void layout(int dim, const int64_t N[3], const double* in, double* out,
       const double* w = v + (end ? 0 : along_y ? nx : nx * ny);
       for (int64_t x = 0; x < nx; ++x) o[x] = v[x] + 0.5 * (w[x] - v[x]);
     }
-  }, nx);
+  }, nx, kLayoutGrain);
 }
 
 }  // namespace kw
@@ -1837,15 +1854,23 @@ int kw_run_noalloc(const kw_problem* prob, kw_outputs* out, char* err, size_t er
   });
 }
 
-int kw_layout(int32_t dim, const int64_t N[3], const double* in, double* out,
-              double* const sg[3], char* err, size_t errlen) {
+int kw_layout_strided(int32_t dim, const int64_t N[3], const int64_t stride[3], const double* in,
+                      double* out, double* const sg[3], char* err, size_t errlen) {
   return kw_guarded(err, errlen, [&]() {
-    if (!N || !in || !out) kw::fail(KW_EINVAL, "NULL argument");
+    if (!N || !stride || !in || !out) kw::fail(KW_EINVAL, "NULL argument");
     if (dim < 1 || dim > 3) kw::fail(KW_EINVAL, "dim must be 1, 2 or 3");
     for (int a = 0; a < dim; ++a)
       if (N[a] < 1) kw::fail(KW_EINVAL, "grid sizes must be positive");
-    kw::layout(dim, N, in, out, sg);
+    kw::layout(dim, N, stride, in, out, sg);
   });
+}
+
+int kw_layout(int32_t dim, const int64_t N[3], const double* in, double* out,
+              double* const sg[3], char* err, size_t errlen) {
+  int64_t stride[3] = {1, 1, 1};
+  if (N)
+    for (int a = dim - 2; a >= 0 && dim <= 3; --a) stride[a] = stride[a + 1] * N[a + 1];
+  return kw_layout_strided(dim, N, stride, in, out, sg, err, errlen);
 }
 
 int kw_smooth(int32_t dim, const int64_t N[3], const double* in, const double* win, double* out,

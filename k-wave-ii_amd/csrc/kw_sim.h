@@ -140,12 +140,18 @@ inline cf round_magnitude(std::complex<double> v) {
 inline double sinc(double x) { return x == 0.0 ? 1.0 : std::sin(x) / x; }
 
 // f(i) for i < n on up to 16 host threads; `work` is the cost of one item in
-// element operations (small loops stay on the calling thread)
+// element operations (small loops stay on the calling thread) and `grain` the
+// least work of a thread
 template <class F>
-void parallel_for(int64_t n, F f, int64_t work = 1) {
+void parallel_for(int64_t n, F f, int64_t work = 1, int64_t grain = 1) {
   int nt = (int)std::thread::hardware_concurrency();
   nt = std::max(1, std::min(nt, 16));
   if (n * work < 100000) nt = 1;
+  nt = (int)std::max<int64_t>(1, std::min<int64_t>(nt, n * work / grain));
+  if (nt == 1) {
+    for (int64_t i = 0; i < n; ++i) f(i);
+    return;
+  }
   std::vector<std::thread> th;
   const int64_t chunk = (n + nt - 1) / nt;
   for (int w = 0; w < nt; ++w) {

@@ -213,8 +213,8 @@ def load(backend: str = "hip") -> C.CDLL:
     lib.kw_sim_destroy.argtypes = [C.c_void_p]
     lib.kw_sim_step_timed.argtypes = [C.c_void_p, C.c_int64, P(C.c_double), P(KernelStats)] + err
     lib.kw_smooth.argtypes = [C.c_int32, P(C.c_int64), c_double_p, c_double_p, c_double_p] + err
-    lib.kw_layout.argtypes = [C.c_int32, P(C.c_int64), c_double_p, c_double_p,
-                              P(c_double_p)] + err
+    lib.kw_layout_strided.argtypes = [C.c_int32, P(C.c_int64), P(C.c_int64), c_double_p,
+                                      c_double_p, P(c_double_p)] + err
     lib.kw_save_problem.argtypes = [P(Problem), C.c_char_p] + err
     lib.kw_run_file.argtypes = [C.c_char_p, C.c_char_p, C.c_uint32, C.c_int64] + err
     lib.kw_engine_create.argtypes = [P(EngineConfig), P(C.c_void_p)] + err
@@ -261,16 +261,21 @@ def as_f64(a):
 
 
 def _layout(a, out, sg):
+    if not a.flags.aligned or any(s % a.itemsize for s in a.strides):
+        a = np.ascontiguousarray(a)
     sgp = None if sg is None else (c_double_p * 3)(*[dptr(s) for s in sg])
-    call(load(active_backend()).kw_layout, C.c_int32(a.ndim),
-         (C.c_int64 * 3)(*a.shape, *([1] * (3 - a.ndim))), dptr(a), dptr(out), sgp)
+    sizes = (C.c_int64 * 3)(*a.shape, *([1] * (3 - a.ndim)))
+    steps = (C.c_int64 * 3)(*[s // a.itemsize for s in a.strides], *([0] * (3 - a.ndim)))
+    call(load(active_backend()).kw_layout_strided, C.c_int32(a.ndim), sizes, steps, dptr(a),
+         dptr(out), sgp)
 
 
 def fortran_flat(a):
     """Column-major (MATLAB) flattening of a grid array as float64; large
-    row-major grids go through the library's threaded transpose."""
+    grids in any other order (row-major, cut out of a larger array, axes
+    exchanged or reversed) go through the library's threaded transpose."""
     a = np.asarray(a, dtype=np.float64)
-    if a.ndim < 2 or a.size < (1 << 16) or not a.flags.c_contiguous:
+    if a.ndim not in (2, 3) or a.size < (1 << 16) or a.flags.f_contiguous:
         return np.ascontiguousarray(a.ravel(order="F"))
     out = np.empty(a.size)
     _layout(a, out, None)
@@ -283,12 +288,9 @@ def fortran_staggered(a):
     a = np.asarray(a, dtype=np.float64)
     if a.size >= (1 << 16):
         sg = [np.empty(a.size) for _ in range(a.ndim)]
-        if a.flags.c_contiguous:
-            flat = np.empty(a.size)
-            _layout(a, flat, sg)
-        else:
-            flat = fortran_flat(a)
-            _layout(flat.reshape(a.shape, order="F"), flat, sg)
+        # (a column-major grid is its own flattening)
+        flat = fortran_flat(a) if a.flags.f_contiguous else np.empty(a.size)
+        _layout(flat.reshape(a.shape, order="F") if a.flags.f_contiguous else a, flat, sg)
         return flat, sg
     sg = []
     for ax in range(a.ndim):

@@ -5,6 +5,8 @@ precision and round once, so an entry differs at most in its last single
 bit, and a few steps at most to 1e-6 of the largest value.  The staggered
 column-major layout of a density map is checked against NumPy bit for bit."""
 
+import itertools
+
 import numpy as np
 import pytest
 
@@ -67,3 +69,53 @@ def test_layout(shape, order):
         want = m.copy()
         want[:-1] = m[:-1] + 0.5 * (m[1:] - m[:-1])
         assert np.array_equal(sg[ax], np.moveaxis(want, 0, ax).ravel(order="F"))
+
+
+def _views(shape):
+    """Grids in the orders that a program's arrays come in, other than C and F."""
+    rng = np.random.default_rng(2)
+    n = len(shape)
+    wide = rng.random(tuple(k + 5 for k in shape))
+    yield "slice", wide[tuple(slice(2, k + 2) for k in shape)]
+    yield "slice_f", np.asfortranarray(wide)[tuple(slice(2, k + 2) for k in shape)]
+    yield "step", rng.random(shape[:-1] + (2 * shape[-1],))[..., ::2]
+    yield "reversed", rng.random(shape)[tuple(slice(None, None, -1) for _ in shape)]
+    yield "one_plane", np.broadcast_to(rng.random(shape[:-1] + (1,)), shape)
+    for p in itertools.permutations(range(n)):
+        if list(p) not in (list(range(n)), list(range(n))[::-1]):
+            yield f"axes{p}", rng.random([shape[i] for i in p]).transpose(np.argsort(p))
+    yield "single", rng.random(shape).astype(np.float32)[:, ::-1]
+    raw = np.zeros(8 * int(np.prod(shape)) + 1, dtype=np.uint8)[1:].view(np.float64).reshape(shape)
+    raw[...] = rng.random(shape)
+    yield "unaligned", raw
+
+
+@pytest.mark.parametrize("shape", [(300, 257), (67, 33, 41), (33, 1, 2000), (1, 70, 1000)])
+def test_layout_of_views(shape, monkeypatch):
+    """Large grids in any order take the threaded transpose and give NumPy's
+    column-major flattening and the same staggered copies."""
+    from kwhip import _abi
+    calls = []
+    inner = _abi._layout
+    monkeypatch.setattr(_abi, "_layout", lambda *a: (calls.append(1), inner(*a))[1])
+    for name, a in _views(shape):
+        calls.clear()
+        with _abi._backend_override("emu"):
+            got = _abi.fortran_flat(a)
+            assert calls or a.flags.f_contiguous, name
+            flat, sg = _abi.fortran_staggered(a)
+        assert np.array_equal(got, a.ravel(order="F")), name
+        assert np.array_equal(flat, a.ravel(order="F")), name
+        d = a.astype(np.float64)
+        for ax in range(a.ndim):
+            m = np.moveaxis(d, ax, 0)
+            want = m.copy()
+            want[:-1] = m[:-1] + 0.5 * (m[1:] - m[:-1])
+            assert np.array_equal(sg[ax], np.moveaxis(want, 0, ax).ravel(order="F")), (name, ax)
+
+
+def test_flattening_takes_more_axes():
+    from kwhip import _abi
+    a = np.random.default_rng(3).random((300, 257, 1, 1))
+    with _abi._backend_override("emu"):
+        assert np.array_equal(_abi.fortran_flat(a), a.ravel(order="F"))
