@@ -101,13 +101,16 @@ static float* source_km(Sim& S, const kw_time_source& src) {
 // 1 / rho0 where they are uniform), the same way in every step: up to 2e-7 in
 // the squared speed of every wave, most of the error of a long run in a
 // uniform medium.  A gradient and a divergence carry the square of kappa per
-// step, so kappa takes the square root of what their product lost.
-static double rounding_of(const kw_problem& pr, double dt) {
-  auto lost = [](double v) { return v / (double)(float)v; };
-  double f = lost(dt) * lost(dt);
-  if (!pr.c0) f *= lost(pr.c0_scalar) * lost(pr.c0_scalar);
-  if (!pr.rho0) f *= lost(pr.rho0_scalar) * lost(1.0 / pr.rho0_scalar);
-  return std::sqrt(f);
+// step, so kappa takes the square root of what their product lost, here with
+// the time step `dt` applied as `applied`.
+static double lost_of(double v, float applied) {
+  const double f = v / (double)applied;
+  return std::fabs(f - 1.0) < 1e-6 ? f : 1.0;
+}
+
+static double rounding_of(const Sim::OpParams& o, double dt, float applied) {
+  const double f = lost_of(dt, applied);
+  return std::sqrt(f * f * o.lost_c0 * o.lost_rho0);
 }
 
 std::unique_ptr<Sim> create_sim(const kw_problem* pr_in, void* stream, Arena* arena) {
@@ -518,7 +521,11 @@ std::unique_ptr<Sim> create_sim(const kw_problem* pr_in, void* stream, Arena* ar
     }
     return std::sqrt(acc);
   };
-  const double fit = rounding_of(*pr, dt);
+  if (!pr->c0) S->op.lost_c0 = std::pow(lost_of(pr->c0_scalar, (float)pr->c0_scalar), 2);
+  if (!pr->rho0)
+    S->op.lost_rho0 = lost_of(pr->rho0_scalar, (float)pr->rho0_scalar) *
+                      lost_of(1.0 / pr->rho0_scalar, (float)(1.0 / pr->rho0_scalar));
+  const double fit = rounding_of(S->op, dt, P.dt);
   const bool dev_tables = S->setup_on_device(G.nspec);
   if (dev_tables) P.kappa = S->setup_table(SETUP_SINC, cref, dt, use_k, 0.0, Ntot / fit);
   else P.kappa = S->spectral_table([&](int ix, int iy, int iz) {
@@ -1260,15 +1267,18 @@ void change_dt(Sim& S, double dt_prev, double dt_new) {
   Sim::DtChange c;
   c.dt_mean = f_mean;
   c.dt_new = f_new;
+  // both kappa tables take up the rounding of the step that they run with, as
+  // that of the first step does
+  const double fit_mean = rounding_of(o, (t1 + t2) / 2, f_mean), fit = rounding_of(o, t2, f_new);
   // setkSpaceCorrection.m:45-53 (NaN, at k = 0, becomes 1)
   c.kappa_mix = S.spectral_table([&](int ix, int iy, int iz) {
-    if (!o.use_k) return 1.0 / Ntot;
+    if (!o.use_k) return fit_mean / Ntot;
     const double ck = o.c_ref * kmag(ix, iy, iz);
     double v = 2.0 * (std::sin(ck * t2 / 2) + std::sin(ck * t1 / 2) * (std::cos(ck * t2 / 2) /
                                                                        std::cos(ck * t1 / 2))) /
                (ck * (t1 + t2));
     if (std::isnan(v)) v = 1.0;
-    return v / Ntot;
+    return v * fit_mean / Ntot;
   });
   if (o.use_k)
     c.ksplit = S.spectral_table([&](int ix, int iy, int iz) {
@@ -1278,7 +1288,7 @@ void change_dt(Sim& S, double dt_prev, double dt_new) {
       return v / Ntot;
     });
   c.kappa_new = S.spectral_table([&](int ix, int iy, int iz) {
-    return (o.use_k ? sinc(o.c_ref * kmag(ix, iy, iz) * t2 / 2) : 1.0) / Ntot;
+    return (o.use_k ? sinc(o.c_ref * kmag(ix, iy, iz) * t2 / 2) : 1.0) * fit / Ntot;
   });
   // setupQuarticPML.m with the mean step (velocity half) and the new step
   auto profile = [&](int a, double dt, bool staggered) {

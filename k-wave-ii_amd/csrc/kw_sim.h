@@ -287,6 +287,9 @@ struct Sim {
     int pml_size[3] = {0, 0, 0};
     double pml_alpha[3] = {0, 0, 0};
     bool use_sg = true, use_k = true;
+    // what single precision loses of a uniform c0 (squared) and of a uniform
+    // rho0 times 1 / rho0
+    double lost_c0 = 1.0, lost_rho0 = 1.0;
   } op;
   // a time-step change armed for the next step: the tables of the
   // transition step's velocity half (mean step) and those of the new step
