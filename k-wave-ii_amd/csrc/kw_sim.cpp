@@ -675,12 +675,15 @@ std::unique_ptr<Sim> create_sim(const kw_problem* pr_in, void* stream, Arena* ar
       P.sens_idx = S->upload(idx);
       // p and u time series of ascending points are written by the x passes
       // (p by x_eos, or by the x_div kernels that do; the 'WSWS-FFT' record of
-      // u swaps its last radial column in after the step); any other point
+      // u swaps its last radial column in after the step, and a nonlinear
+      // 'WSWA-FFT' one rewrites the copies 2-4 of p); any other point
       // statistic needs the point kernel, which then writes them all
       uint32_t by_rows = KW_REC_U;
       if (P.eos == EOS_ABSORBING || x_div_records(G.dim, S->fixed_len(PK_X_DIV)))
         by_rows |= KW_REC_P;
-      if (P.rec_points && (P.rec_points & ~by_rows) == 0 && !S->as_ws &&
+      const bool rewritten = S->axisym && P.nonlinear &&
+                             *std::max_element(idx.begin(), idx.end()) >= G.Ny / 4 * G.Nx;
+      if (P.rec_points && (P.rec_points & ~by_rows) == 0 && !S->as_ws && !rewritten &&
           std::is_sorted(idx.begin(), idx.end())) {
         std::vector<int32_t> rows(G.nrows + 1);
         for (int64_t r = 0, k = 0; r <= G.nrows; ++r) {
