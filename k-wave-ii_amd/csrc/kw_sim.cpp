@@ -654,6 +654,7 @@ std::unique_ptr<Sim> create_sim(const kw_problem* pr_in, void* stream, Arena* ar
     P.tr_data = S->upload_map(pr->time_reversal_boundary_data, S->nsens * pr->Nt);
   }
   // sensor outputs
+  std::vector<int32_t> rows;  // first point of each row, where the x passes record
   if (S->nsens > 0 && !S->time_rev) {
     if (interp) {
       // record.tri / record.bc, column-major [points x (dim+1)], stored
@@ -685,14 +686,11 @@ std::unique_ptr<Sim> create_sim(const kw_problem* pr_in, void* stream, Arena* ar
                              *std::max_element(idx.begin(), idx.end()) >= G.Ny / 4 * G.Nx;
       if (P.rec_points && (P.rec_points & ~by_rows) == 0 && !S->as_ws && !rewritten &&
           std::is_sorted(idx.begin(), idx.end())) {
-        std::vector<int32_t> rows(G.nrows + 1);
+        rows.resize((size_t)G.nrows + 1);
         for (int64_t r = 0, k = 0; r <= G.nrows; ++r) {
           while (k < S->nsens && (int64_t)idx[k] < r * G.Nx) ++k;
           rows[r] = (int32_t)k;
         }
-        P.row_sens = S->upload(rows);
-        P.rec_rows = P.rec_points;
-        P.rec_points = 0;
       }
     }
     if (directivity && (S->record & KW_REC_P)) {
@@ -827,6 +825,14 @@ std::unique_ptr<Sim> create_sim(const kw_problem* pr_in, void* stream, Arena* ar
   };
   prep(pr->p_source, P.srcp, S->p_grid);
   for (int a = 0; a < dim; ++a) prep(pr->u_source[a], P.srcu[a], S->u_grid[a]);
+  // last, so that a simulation which fills its arena without the row table
+  // keeps the point kernel
+  if (!rows.empty() && S->has_room<int32_t>(rows.size())) {
+    P.row_sens = S->upload(rows);
+    P.rec_rows = P.rec_points;
+    P.rec_points = 0;
+    changed = true;
+  }
   if (changed) dev_h2d(S->dP, &S->P, sizeof(ProbDev), S->stream);
   S->end_staging();
   dev_sync(S->stream);

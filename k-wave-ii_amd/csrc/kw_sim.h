@@ -342,12 +342,17 @@ struct Sim {
     if (own_stream) dev_stream_destroy(stream);
   }
 
+  static size_t arena_bytes(size_t nb) { return ((nb ? nb : 1) + 255) / 256 * 256; }
+  template <class T>
+  bool has_room(size_t n) const {
+    return !arena || arena_bytes(n * sizeof(T)) <= arena->size - arena->used;
+  }
   template <class T>
   T* alloc(size_t n) {
     const size_t nb = n * sizeof(T);
     void* p;
     if (arena) {
-      const size_t need = ((nb ? nb : 1) + 255) / 256 * 256;
+      const size_t need = arena_bytes(nb);
       if (need > arena->size - arena->used)
         fail(KW_ENOMEM, "the problem needs more device memory than the " +
                             std::to_string(arena->size >> 20) +
