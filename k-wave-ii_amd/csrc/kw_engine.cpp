@@ -348,8 +348,8 @@ struct Group {
       // threads per pencil of the engine that serves the launch
       const Geometry& g = sims[i]->G;
       const int Nl = dim == 3 ? g.Nz : g.Ny;
-      hp[i].Gl = fixed[2] ? strided_threads(Nl) : rt_threads(Nl);
-      if (dim == 3) hp[i].Gy = fixed[1] ? y_threads(g.Ny) : rt_threads(g.Ny);
+      hp[i].Gl = fixed[2] ? fixed_plan(Nl).strided : rt_threads(Nl);
+      if (dim == 3) hp[i].Gy = fixed[1] ? fixed_plan(g.Ny).y : rt_threads(g.Ny);
     }
     probs = (ProbDev*)dev_alloc(sizeof(ProbDev) * n);
     live.push_back(probs);

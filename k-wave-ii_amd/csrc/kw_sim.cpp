@@ -313,8 +313,8 @@ std::unique_ptr<Sim> create_sim(const kw_problem* pr_in, void* stream, Arena* ar
   S->tiles = choose_tiles(*pr, S->stream, arena == nullptr);
   S->plan_launches();
   P.fx = S->make_plan(G.Nx);
-  P.fy = S->make_plan(G.Ny);
-  P.fz = dim == 3 ? S->make_plan(G.Nz) : P.fy;
+  P.fy = G.Ny == G.Nx ? P.fx : S->make_plan(G.Ny);
+  P.fz = dim != 3 || G.Nz == G.Ny ? P.fy : G.Nz == G.Nx ? P.fx : S->make_plan(G.Nz);
 
   // medium (rounded once from double)
   const int64_t n = G.ncell;
@@ -680,7 +680,8 @@ std::unique_ptr<Sim> create_sim(const kw_problem* pr_in, void* stream, Arena* ar
       // 'WSWA-FFT' one rewrites the copies 2-4 of p); any other point
       // statistic needs the point kernel, which then writes them all
       uint32_t by_rows = KW_REC_U;
-      if (P.eos == EOS_ABSORBING || x_div_records(G.dim, S->fixed_len(PK_X_DIV)))
+      const int fx = S->fixed_len(PK_X_DIV);
+      if (P.eos == EOS_ABSORBING || G.dim == 2 || fx == 0 || fixed_plan(fx).x_div_3d)
         by_rows |= KW_REC_P;
       const bool rewritten = S->axisym && P.nonlinear &&
                              *std::max_element(idx.begin(), idx.end()) >= G.Ny / 4 * G.Nx;

@@ -92,6 +92,28 @@ inline int stage_length(int N) {
 // threads per pencil of the runtime engine, from the length its stages run at
 inline int rt_threads(int N) { return stage_threads(stage_length(N)); }
 
+// Threads per pencil of the strided and y passes of the fixed lengths, and
+// whether their x_div records, from constants: the plan search takes up to
+// 60 us a length at run time, for every simulation and every member of a group
+// whose tables are made again.
+struct FixedPlan {
+  int strided, y;
+  bool x_div_3d;
+};
+inline FixedPlan fixed_plan(int N) {
+  switch (N) {
+#define KW_FIXED_PLAN(S)                                                                   \
+  case S: {                                                                                \
+    constexpr FixedPlan p{strided_threads(S), y_threads(S), x_div_records(3, S)};          \
+    return p;                                                                              \
+  }
+    KW_FIXED_SIZES_ALL(KW_FIXED_PLAN)
+    KW_FIXED_SIZES_XL(KW_FIXED_PLAN)
+#undef KW_FIXED_PLAN
+  }
+  return FixedPlan{strided_threads(N), y_threads(N), x_div_records(3, N)};
+}
+
 // wavenumber of ifftshifted index i (kWaveGrid.m:779-797 then ifftshift):
 // (2 pi/d) * (n/N) with n = i for i < ceil(N/2), else i - N
 inline double kvec(int i, int N, double d) {
@@ -121,14 +143,20 @@ inline cf round_magnitude(std::complex<double> v) {
   const double c = v.real(), s = v.imag(), r = std::abs(v);
   cf best{(float)c, (float)s};
   if (std::fabs(c) < 1e-7 * r || std::fabs(s) < 1e-7 * r) return best;
+  // (a nextafter, a hypot and a division for each pair took 480 us for 1024
+  // twiddles, as long as the rest of a small simulation's creation; 115 so)
+  const double half = 0.5 / r, tenth = 0.1 / r, r2 = r * r;
+  float xs[3], ys[3];
+  for (int i = 0; i < 3; ++i) {
+    xs[i] = i == 1 ? best.x : std::nextafter(best.x, (i - 1) * 1e30f);
+    ys[i] = i == 1 ? best.y : std::nextafter(best.y, (i - 1) * 1e30f);
+  }
   double least = 1e300;
-  for (int i = -1; i <= 1; ++i)
-    for (int j = -1; j <= 1; ++j) {
-      const float x = i == 0 ? (float)c : std::nextafter((float)c, i * 1e30f);
-      const float y = j == 0 ? (float)s : std::nextafter((float)s, j * 1e30f);
-      const double m = std::hypot((double)x, (double)y) - r;
-      const double t = ((double)y * c - (double)x * s) / r;
-      const double e = std::fabs(m) + 0.1 * std::fabs(t);
+  for (const float x : xs)
+    for (const float y : ys) {
+      const double m = ((double)x * x + (double)y * y - r2) * half;
+      const double t = ((double)y * c - (double)x * s) * tenth;
+      const double e = std::fabs(m) + std::fabs(t);
       if (e < least) {
         least = e;
         best = cf{x, y};
@@ -672,7 +700,7 @@ struct Sim {
     // pencil, which a group of uneven sizes uses: see Group::rebuild)
     // strided y pass (3D): <= 1024 threads, LDS Ny twiddles + P*(Ny+1)
     if (G.dim == 3) {
-      const int Gy = fixed_len(PK_YFWD) ? y_threads(G.Ny) : Gof(G.Ny);
+      const int Gy = fixed_len(PK_YFWD) ? fixed_plan(G.Ny).y : Gof(G.Ny);
       const int Ly = stage_length(G.Ny);
       int P = std::max(1, std::min(pencils_env("KW_PENCILS_Y", tiles.y ? tiles.y : 16),
                                    1024 / std::max(Gy, Gof(G.Ny))));
@@ -689,7 +717,7 @@ struct Sim {
     // last-axis pass: <= 1024 threads, LDS N twiddles + 2*P*N
     {
       const int Nl = G.dim == 3 ? G.Nz : G.Ny;
-      const int Gl = fixed_len(PK_SPEC) ? strided_threads(Nl) : Gof(Nl);
+      const int Gl = fixed_len(PK_SPEC) ? fixed_plan(Nl).strided : Gof(Nl);
       const int Ll = stage_length(Nl);
       int P = std::max(1, std::min(pencils_env("KW_PENCILS_L", tiles.l ? tiles.l : 16),
                                    1024 / std::max(Gl, Gof(Nl))));
