@@ -261,6 +261,7 @@ struct Ticket;
 
 struct Group {
   int dim = 0;
+  int comp = 0;  // velocity components, the most of any member
   bool absorbing = false;
   bool axisym = false;  // axisymmetric members: stepped one by one
   void* stream = nullptr;
@@ -390,7 +391,9 @@ struct Group {
       dev_h2d(tiles[k], start.data(), sizeof(int32_t) * n, stream);
     }
     any_points = any_grid = false;
+    comp = 0;
     for (Sim* s : sims) {
+      comp = std::max(comp, (int)s->P.dim);
       any_points = any_points || s->P.rec_points != 0;
       any_grid = any_grid || s->P.rec_grid != 0;
     }
@@ -404,7 +407,7 @@ struct Group {
     const int fx = fixed[k == GX ? 0 : (k == GY ? 1 : 2)];
     PassArgs a = a0;
     int nb = geo[k].nb;
-    const int split = split_buffers(kind, a, dim, (int64_t)nb * geo[k].T);
+    const int split = split_buffers(kind, a, dim, comp, (int64_t)nb * geo[k].T);
     if (split > 1) {
       a.ysplit = nb;
       nb *= split;

@@ -438,9 +438,11 @@ KW_HOSTDEV bool spec_is_aux(const PassArgs& A) { return A.mode == SM_SHIFT || A.
 // code.
 template <class LS, bool AUX, class Ctx>
 KW_BODY void body_spec(Ctx& c, const Batch& B, const PassArgs& A) {
-  // SM_DIV and SM_ABS with ysplit: one buffer per block
+  // SM_DIV and SM_ABS with ysplit: one buffer per block (a 1-D problem in a
+  // launch with 2-D ones has no second component)
   int tile, b0;
   const ProbDev& P = split_prob(c, B, A, tile, b0);
+  if (A.mode == SM_DIV && b0 >= P.dim) return;
   if (b0 == 0) advance_step(P, A, tile, c.tid());
   const bool d3 = P.dim == 3;
   const FftPlan& pl = d3 ? P.fz : P.fy;

@@ -243,11 +243,13 @@ inline size_t launch_lds(PassKind k, int fixed, const PassArgs& a, size_t full) 
 // about four wavefronts per SIMD a block's buffers one after another are its
 // latency, above that the split only repeats its set-up and table reads.
 constexpr int64_t kSplitThreads = 256 * 4 * 64 * 4;
-inline int split_buffers(PassKind k, const PassArgs& a, int dim, int64_t threads) {
+// `comp` is the problem's number of velocity components; a 1-D problem, whose
+// grid has two axes, has one.
+inline int split_buffers(PassKind k, const PassArgs& a, int dim, int comp, int64_t threads) {
   if (k == PK_YFWD || k == PK_YINV) return a.nbuf;
   if (threads >= kSplitThreads) return 1;
   if (k == PK_X_GRAD) return dim;
-  if (k == PK_SPEC && a.mode == SM_DIV) return dim;
+  if (k == PK_SPEC && a.mode == SM_DIV) return comp;
   if (k == PK_SPEC && a.mode == SM_ABS) return 2;
   return 1;
 }
@@ -568,7 +570,7 @@ struct Sim {
     const int fx = fixed_len(k);
     PassArgs a = a0;
     int nb = g->nb;
-    const int split = split_buffers(k, a, G.dim, (int64_t)nb * g->T);
+    const int split = split_buffers(k, a, G.dim, P.dim, (int64_t)nb * g->T);
     if (split > 1) {
       a.ysplit = nb;
       nb *= split;
