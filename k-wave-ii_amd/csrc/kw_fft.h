@@ -114,8 +114,8 @@ KW_HOSTDEV constexpr int strided_threads(int N, int most = 12) {
   }
   return g;
 }
-// The y passes of an axis above 256: at most eight elements per thread.  Their
-// blocks have 768 threads and more, of which a CU holds two only while a
+// The y passes of an axis above 256 (384 is the only such length with a fixed y
+// pass): at most eight elements per thread.  Their blocks have 768 threads and more, of which a CU holds two only while a
 // thread's registers are few (384 = 12 8 4 on 48 threads: 224 us a forward
 // launch of 384^3, 167 as 8 8 6 on 64).
 KW_HOSTDEV constexpr int y_most(int N) { return N > 256 && strided_threads(N, 8) > 0 ? 8 : 12; }
@@ -305,6 +305,8 @@ KW_BODY void dft<5, true>(cf* v) { dft5<true>(v); }
 
 // odd prime radix from the pairs a_k = v_k + v_(R-k), b_k = v_k - v_(R-k):
 // X_j = v_0 + sum_k cos(2 pi jk/R) a_k -+ i sum_k sin(2 pi jk/R) b_k
+// (Rounded to single, without remainders: a stage of radix 13 holds 12 constants
+// already, the runtime engine has no registers for twice as many.)
 template <int R>
 struct PrimeTrig;  // cos and sin of 2 pi m / R, m = 1 .. (R - 1) / 2
 template <>
@@ -804,15 +806,12 @@ struct PlanRt {
   }
 };
 
-// threads per pencil of the runtime engine: ceil(N / KW_E)
-KW_HOSTDEV constexpr int ct_threads(int N) { return (N + KW_E - 1) / KW_E; }
-
 // threads per pencil of the fixed-length x passes: the smallest power of two
-// that leaves a thread at most six elements, so that every pencil lies in one
-// wavefront and the stages synchronise with wavefront barriers instead of
+// with at most six elements of the pencil each, so that every pencil lies in
+// one wavefront and the stages synchronise with wavefront barriers instead of
 // block barriers (the extra lanes idle in stages with fewer butterflies than
 // lanes); lengths above 384 take a wavefront per 256 elements (one step of 600
-// points 37 -> 29 us against ceil(N / KW_E))
+// points 37 -> 29 us against N / 8 threads)
 KW_HOSTDEV constexpr int x_threads(int N) {
   for (int p = 1; p <= 64; p <<= 1)
     if (6 * p >= N) return p;

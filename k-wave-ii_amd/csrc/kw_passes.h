@@ -105,7 +105,7 @@ KW_BODY XTile x_tile(Ctx& c, const ProbDev& P, int tile) {
 }
 
 // the twiddles into LDS and the block barrier that makes them visible to
-// every wavefront; the caller has issued its first loads before
+// every wavefront, before any load of the pass
 template <class Ctx>
 KW_BODY void x_start(Ctx& c, const ProbDev& P) {
   put_twiddles(c, P.fx, c.lds());
@@ -296,9 +296,9 @@ KW_BODY void advance_step(const ProbDev& P, const PassArgs& A, int tile, int tid
 
 template <bool INV, class YS, class Ctx>
 KW_BODY void body_ypass(Ctx& c, const Batch& B, const PassArgs& A) {
+  // one buffer per block (split_buffers)
   int tile, b0;
   const ProbDev& P = split_prob(c, B, A, tile, b0);
-  const int b1 = A.ysplit > 0 ? b0 + 1 : A.nbuf;
   if (b0 == 0) advance_step(P, A, tile, c.tid());
   const int N = P.Ny, G = P.Gy, Pn = P.Py;
   // LDS: the L twiddles, then the pencils (L elements each: the length the
@@ -336,21 +336,15 @@ KW_BODY void body_ypass(Ctx& c, const Batch& B, const PassArgs& A) {
     stride = 1;
     lds = LdsPencils{lp + (int64_t)p * (L + 1), 0, 1, false};
   }
-  for (int b = b0; b < b1; ++b) {
-    cf* S = P.S[A.buf[b]];
-    auto ld = [&](int, int n) -> cf { return KW_LD32(S, base + (uint32_t)n * stride); };
-    auto st = [&](int, int n, cf v, int) { KW_ST32(S, base + (uint32_t)n * stride, v); };
-    if (b == b0) {
-      // the first transform's loads are in flight while the twiddles come
-      typename YS::template Pre<decltype(ld)> pre;
-      YS::load_first(g, ld, pre);
-      put_twiddles(c, P.fy, c.lds());
-      if (YS::twiddles_first) c.sync();
-      YS::template fft_pre<1, INV>(c, P.fy, tw, g, G, active, ld, pre, st, lds);
-    } else {
-      YS::template fft_tw<1, INV>(c, P.fy, tw, g, G, active, ld, st, lds);
-    }
-  }
+  cf* S = P.S[A.buf[b0]];
+  auto ld = [&](int, int n) -> cf { return KW_LD32(S, base + (uint32_t)n * stride); };
+  auto st = [&](int, int n, cf v, int) { KW_ST32(S, base + (uint32_t)n * stride, v); };
+  // the transform's loads are in flight while the twiddles come
+  typename YS::template Pre<decltype(ld)> pre;
+  YS::load_first(g, ld, pre);
+  put_twiddles(c, P.fy, c.lds());
+  if (YS::twiddles_first) c.sync();
+  YS::template fft_pre<1, INV>(c, P.fy, tw, g, G, active, ld, pre, st, lds);
 }
 
 // ---------------------------------------------------------------------------

@@ -76,8 +76,9 @@ def test_emu_parity_3d(name):
     # the velocity split's last-axis pass on fixed-length kernels
     (2, "u_split", (30, 64)),
     (3, "u_split", (12, 16, 64)),
-    # lengths with a prime factor above 7 (Bluestein's chirp-z transform on
-    # every axis kind): 22 = 2 x 11, 26 = 2 x 13, 34 = 2 x 17, 31 prime
+    # lengths with a prime factor above 7 on every axis kind: 22 = 2 x 11 and
+    # 26 = 2 x 13 run directly, 34 = 2 x 17 and 31 as Bluestein's chirp-z
+    # transform
     (1, "p0_hetero_absorbing", (22,)),
     (1, "time_reversal", (31,)),
     (2, "p0_hetero_absorbing", (22, 26)),

@@ -69,7 +69,8 @@ def test_parity_3d_sizes(name, shape, hip_lib):
 
 
 @pytest.mark.parametrize("dim,name,shape", [
-    # lengths with a prime factor above 7: Bluestein's chirp-z transform
+    # lengths with a prime factor above 7: 13, 22 and 26 run directly, 31 and
+    # 34 as Bluestein's chirp-z transform
     (1, "p0_hetero_absorbing", (22,)),
     (2, "p0_hetero_absorbing", (22, 26)),
     (2, "time_reversal", (34, 31)),
