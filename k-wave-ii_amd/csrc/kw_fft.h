@@ -70,10 +70,11 @@ constexpr int kStageCost = 3;
 // elements of one stage of radix R per thread
 KW_HOSTDEV constexpr int ct_stage_work(int N, int R, int G) { return (N / R + G - 1) / G * R; }
 
+// `slots`: some stage leaves a thread at most that many elements
 KW_HOSTDEV constexpr void ct_search(int N, int rest, int G, int emax, CtPlan cur, int cost, int top,
-                         CtPlan& best) {
+                         CtPlan& best, int slots = 1 << 20, int least = 1 << 20) {
   if (rest == 1) {
-    if (cur.nst > 0 && cost < best.cost) {
+    if (cur.nst > 0 && cost < best.cost && least <= slots) {
       best = cur;
       best.cost = cost;
     }
@@ -88,7 +89,8 @@ KW_HOSTDEV constexpr void ct_search(int N, int rest, int G, int emax, CtPlan cur
     if (w > emax) continue;
     CtPlan nx = cur;
     nx.r[nx.nst++] = R;
-    ct_search(N, rest / R, G, emax, nx, cost + w + kStageCost, R, best);
+    ct_search(N, rest / R, G, emax, nx, cost + w + kStageCost, R, best, slots,
+              w < least ? w : least);
   }
 }
 
@@ -120,11 +122,16 @@ KW_HOSTDEV constexpr int strided_threads(int N, int most = 12) {
 // launch of 384^3, 167 as 8 8 6 on 64).
 KW_HOSTDEV constexpr int y_most(int N) { return N > 256 && strided_threads(N, 8) > 0 ? 8 : 12; }
 KW_HOSTDEV constexpr int y_threads(int N) { return strided_threads(N, y_most(N)); }
-// x plan: the stage that leaves a thread the fewest elements last, the
-// largest of the others first
+// x plan: the stage that leaves a thread the fewest elements last, at most
+// kXSlots, the largest of the others first.  The x passes keep several values
+// per element in registers; with the plan of least work alone 72, 80 and 648
+// left eight elements and 81, 90, 729 and 810 nine: x_div of 80 x 240 x 240
+// 75 us as 10 8, 42 as 8 5 2, a step 281 -> 234; 648 x 96 x 96 396 -> 325.  The
+// stages more cost small grids of 81 and 90 points (90 x 90 35 -> 38 us a step).
+constexpr int kXSlots = 6;
 KW_HOSTDEV constexpr CtPlan ct_xplan(int N, int G) {
   CtPlan p;
-  ct_search(N, N, G, 12, CtPlan{}, 0, 10, p);
+  ct_search(N, N, G, 12, CtPlan{}, 0, 10, p, kXSlots);
   int last = 0;
   for (int s = 1; s < p.nst; ++s)
     if (ct_stage_work(N, p.r[s], G) <= ct_stage_work(N, p.r[last], G)) last = s;
@@ -877,7 +884,7 @@ using PlanCtY = PlanFixed<CtShape<N, y_threads(N), false, y_most(N)>>;
 // the plan of the x passes for a fixed length
 template <int N>
 struct PlanCtX : PlanFixed<CtShape<N, x_threads(N), true>> {
-  static_assert(CtShape<N, x_threads(N), true>::last_slots <= kMaxSlots, "slot bound");
+  static_assert(CtShape<N, x_threads(N), true>::last_slots <= kXSlots, "slot bound");
 };
 
 }  // namespace kw
