@@ -676,13 +676,19 @@ struct Sim {
     // fixed-length x kernels run x_threads(Nx) threads per pencil
     {
       // (a power of two up to 64 keeps every pencil in one wavefront, whose
-      // barriers cost less than the idle lanes)
+      // barriers cost less than the idle lanes: up to half of them more, or
+      // any number while the launch does not fill the device.  Runtime lengths,
+      // a step with the pencil's own threads and rounded: 77 x 240 x 200 with
+      // 11 or 16 360 and 326 us, 66 x 64 x 64 with 9 or 16 99 and 87; but 139 x
+      // 240 x 200 with 36 or 64 972 and 1236, 159 x 128 x 128 with 40 or 64 418
+      // and 435, 130 x 240 x 200 with 17 or 32 506 and 556)
+      const int64_t pairs = (G.nrows + 1) / 2;
       int Gx = fixed_len(PK_X_GRAD) ? x_threads(G.Nx) : Gof(G.Nx);
-      for (int p = 1; p <= 64 && Gx <= 64; p <<= 1)
-        if (p >= Gx) {
-          Gx = p;
-          break;
-        }
+      if (Gx <= 64) {
+        int p = 1;
+        while (p < Gx) p <<= 1;
+        if (2 * p <= 3 * Gx || pairs * p <= kSplitThreads) Gx = p;
+      }
       const int Lx = stage_length(G.Nx);
       const size_t pencil = sizeof(cf) * (size_t)kNPX * x_lds_stride(Lx);
       const size_t twb = sizeof(cf) * (size_t)Lx;
@@ -692,8 +698,7 @@ struct Sim {
       P = std::max(1, std::min(P, capP));
       this->P.Gx = Gx;
       this->P.Px = P;
-      const int64_t npairs = (G.nrows + 1) / 2;
-      lx.nb = (int)((npairs + P - 1) / P);
+      lx.nb = (int)((pairs + P - 1) / P);
       lx.T = P * Gx;
       lx.lds = pencil * (size_t)P + twb;
       if (Gx > 512 || lx.lds > maxl) fail(KW_EUNSUP, "grid size Nx too large for the x pass");

@@ -52,3 +52,11 @@ def test_lengths_emu(n):
 def test_lengths_hip(n, hip_lib):
     for shape in _shapes(n, n in ALL):
         _check(hip_lib, shape)
+
+
+# runtime lengths of x whose threads per pencil are a power of two in small
+# launches and the length's own number in these
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(139, 130, 64), (66, 260, 130), (74, 130, 130)])
+def test_runtime_lengths_in_large_launches_hip(shape, hip_lib):
+    _check(hip_lib, shape)
