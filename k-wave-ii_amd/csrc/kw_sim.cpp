@@ -403,17 +403,14 @@ std::unique_ptr<Sim> create_sim(const kw_problem* pr_in, void* stream, Arena* ar
       const double an = pr->alpha_coeff_scalar * conv;
       SetupArgs a{};
       a.kind = SETUP_C0;
-      for (float*& o : a.out) o = S->alloc<float>((size_t)n);
+      for (int o = 0; o < (P.eos == EOS_ABSORBING ? 3 : 2); ++o) a.out[o] = S->alloc<float>((size_t)n);
       a.tau = no_abs ? 0.0 : s_tau * (-2.0 * an);
       a.tau_expo = P.eos == EOS_STOKES ? 1.0 : y - 1;
       a.eta = no_disp || P.eos == EOS_STOKES ? 0.0 : s_eta * (2.0 * an * std::tan(kPi * y / 2));
       a.eta_expo = y;
       P.c0 = Field{a.out[0], ~0u};
       P.tau = Field{a.out[1], ~0u};
-      if (P.eos == EOS_ABSORBING)
-        P.eta = Field{a.out[2], ~0u};
-      else
-        S->release(a.out[2]), a.out[2] = nullptr;
+      if (P.eos == EOS_ABSORBING) P.eta = Field{a.out[2], ~0u};
       S->setup_map(pr->c0, n, a);
     } else if (pr->alpha_coeff || pr->c0) {
       std::vector<float> tv(n), ev(n);
